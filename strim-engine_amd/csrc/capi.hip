@@ -207,13 +207,16 @@ int run_group(strim_ctx* ctx, hipStream_t st, Args& a, int nb, bool probs,
     else need_fin = true;
   }
   if (gq) need_fin = true;
-  // k_final decides the general-q draft rows left to the exact resolution: the filtered
-  // ones, and (icdf draws) those whose residual bin overflows
-  bool need_final = gq && a.noise_mode == STRIM_NOISE_ICDF;
+  // general-q draft rows: k_finalize decides the greedy and the fast ones; the unfiltered
+  // ones take the residual draw; k_final decides those left to the exact resolution, the
+  // other filtered ones and (icdf draws) those whose residual bin overflows
+  bool need_qres = false, need_final = false;
   if (gq)
     for (int i = 0; i < nb; ++i) {
-      const strim_sampling_params& q = a.p[i];
-      if ((q.top_k > 0 && q.top_k < a.V) || q.top_p < 1.0f || q.min_p > 0.0f) need_final = true;
+      if (row_class(a.p[i], a.V) != CLS_GENERAL) continue;
+      const bool unf = nofilter(a.p[i], a.V);
+      if (unf) need_qres = true;
+      if (!unf || a.noise_mode == STRIM_NOISE_ICDF) need_final = true;
     }
   // rows per XCD when every chunk reads a history and no general row's cost depends on
   // its mask density (measured: -25 % of k_stream's HBM bytes at cfg2 at equal time;
@@ -237,7 +240,7 @@ int run_group(strim_ctx* ctx, hipStream_t st, Args& a, int nb, bool probs,
     timed(ctx, KID_GFINAL, [&](hipEvent_t e0, hipEvent_t e1) {
       keep(launch_gfinal(a, st, e0, e1));
     });
-  if (a.verify && a.dlog != nullptr) {
+  if (need_qres) {
     // the residual draw of unfiltered general-q rows (rows in other phases return)
     const dim3 grid_r((unsigned)a.R);
     timed(ctx, KID_QRES, [&](hipEvent_t e0, hipEvent_t e1) {

@@ -6,8 +6,10 @@
 //                    min-p on the row maximum, a radix select of the k-th key, a sort of
 //                    the survivors, the top-p cut and the draw, all in LDS;
 //   unfiltered Gumbel rows  from the chunks' two best scores;
-//   general-q draft rows    checked and handed to the residual draw (qres_kernels.hip)
-//                    or k_final's exact resolution.
+//   general-q draft rows    checked; fast rows draw their residual max(0, p - q) here, over
+//                    the kept candidates (q is read for those alone); unfiltered rows are
+//                    handed to the residual draw (qres_kernels.hip), the other general
+//                    rows to k_final's exact resolution.
 // The other general rows are k_gfinal's (gfinal_kernels.hip), which runs beside it.
 // A row whose candidates do not fit the LDS finalize is decided here by the exact
 // streaming resolution (exact.hpp).
@@ -51,6 +53,8 @@ struct FinalShared {
   double d[FTPB / WAVE];
   uint64_t u[FTPB / WAVE];
   int misc[8];
+  double qz;  // general-q draft rows: the draft distribution's sum and maximum
+  float qmq;
   // the exact streaming resolution (rows whose candidates overflow): its histogram
   // masses and gathered buckets use key[] (XB entries)
   uint32_t xhc[XB];
@@ -69,7 +73,8 @@ __device__ __forceinline__ int dbin(float m, float l, float scale) {
 // Decides a row whose candidates overflow the finalize by the exact streaming
 // resolution (all threads of the workgroup call it). Inlined: only exact_row is an
 // out-of-line call, taking the few launch fields it needs by value, so the 3 KB launch
-// block is never copied to private memory.
+// block is never copied to private memory. GQ: see k_finalize.
+template <bool GQ>
 __device__ __forceinline__ void finalize_exact(const Args& a, int r, int b, int j,
                                             const RowParams& p, float m, int arg, int draft,
                                             bool vdr, float l_draft, FinalShared& S) {
@@ -91,9 +96,14 @@ __device__ __forceinline__ void finalize_exact(const Args& a, int r, int b, int 
   xa.drafts = a.drafts;
   xa.noise = a.noise;
   xa.noise_stride = a.noise_stride;
-  xa.has_q = 0;  // general-q rows are decided by k_final
+  xa.has_q = GQ && vdr ? 1 : 0;
   __syncthreads();
-  const XOut xo = exact_row<FTPB, false>(xa, r, b, j, p, m, arg, draft, vdr, l_draft, xs,
+  if (GQ && vdr) {
+    xa.q = q_base(a, b * a.k + j);
+    xa.q.mq = S.qmq;
+    xa.q.Z = S.qz;
+  }
+  const XOut xo = exact_row<FTPB, GQ>(xa, r, b, j, p, m, arg, draft, vdr, l_draft, xs,
                                   *(lds_t<XState>*)&S.x);
   finish_row(a, r, xo.status, xo.token, xo.accept, xo.sig, m, xo.last_key, PH_DONE);
 }
@@ -165,6 +175,7 @@ struct ExactReq {
   float l_draft;
 };
 
+template <bool GQ>
 __device__ __forceinline__ ExactReq finalize_row(const Args& a, int r, int b, int j,
                                                  const RowParams& p, const RowPre& pf,
                                                  FinalShared& S) {
@@ -248,7 +259,9 @@ __device__ __forceinline__ ExactReq finalize_row(const Args& a, int r, int b, in
     finish_row(a, r, STRIM_OK, arg, vdr && arg == draft, 1.0, m, 0ull, PH_DONE);
     return done;
   }
-  if (vdr && a.dlog) {
+  XQ xq;  // (general-q draft rows: their q, valid in wave 0)
+  const bool gq = GQ && vdr;
+  if (gq) {
     // general-q draft row: the draft distribution from k_qprep's slices (its maximum, the
     // draft's table index, fp64 Z = sum exp(v - mq)), published for the residual draw;
     // the draft must be in a valid table (the first draft row's slices checked it)
@@ -268,14 +281,22 @@ __device__ __forceinline__ ExactReq finalize_row(const Args& a, int r, int b, in
       const QPart& pq = pp[lane < QSPLIT ? lane : 0];
       z = wave_sum(lane < QSPLIT && pq.m > -INFINITY ? pq.z * exp((double)pq.m - (double)mq)
                                                      : 0.0);
-      if (t == 0) a.s.qst[qr] = QStat{mq, td, z};
+      if (t == 0) {
+        a.s.qst[qr] = QStat{mq, td, z};
+        S.qz = z;
+        S.qmq = mq;
+      }
     }
     if (bad || td < 0) {
       finish_row(a, r, STRIM_EINVAL, -1, 0, 0.0, m, 0ull, PH_DONE);
       return done;
     }
-    // unfiltered rows: the grid-wide residual draw (qres_kernels.hip); the others: k_final's
-    // exact resolution (the row's first maximum is kept as the fallback token)
+    xq = q_base(a, qr);
+    xq.mq = mq;
+    xq.Z = z;
+    // fast rows go on to the candidates below. Unfiltered rows: the grid-wide residual draw
+    // (qres_kernels.hip); the others: k_final's exact resolution (the row's first maximum
+    // is kept as the fallback token)
     const bool unfiltered = !(p.top_k > 0 && p.top_k < V) && !(p.top_p < 1.0f) && !(p.min_p > 0.0f);
     uint64_t wq = 0ull;
     if (unfiltered && own) {
@@ -286,7 +307,7 @@ __device__ __forceinline__ ExactReq finalize_row(const Args& a, int r, int b, in
       wq = (unsigned long long)__double2ull_rn(wc * XFIX);
       a.s.qpart[(size_t)qr * a.s.wmax + t] = wq;
     }
-    if (unfiltered && a.qskip) {
+    if (p.cls != CLS_FAST && unfiltered && a.qskip) {
       // Only (accepted, token) is asked for: the accept test runs here, on the same
       // numbers as the residual pick's (the row mass is the integer sum of the chunk masses above),
       // so the residual draw runs only for a sequence's first rejected row.
@@ -316,8 +337,10 @@ __device__ __forceinline__ ExactReq finalize_row(const Args& a, int r, int b, in
       }
       return done;
     }
-    finish_row(a, r, STRIM_OK, arg, 0, 0.0, m, 0ull, unfiltered ? PH_QRES : PH_EXACT);
-    return done;
+    if (p.cls != CLS_FAST) {
+      finish_row(a, r, STRIM_OK, arg, 0, 0.0, m, 0ull, unfiltered ? PH_QRES : PH_EXACT);
+      return done;
+    }
   }
   const bool topk = p.top_k > 0 && p.top_k < V;
   const bool topp = p.top_p < 1.0f;
@@ -325,7 +348,7 @@ __device__ __forceinline__ ExactReq finalize_row(const Args& a, int r, int b, in
   const bool by_rank = (p.flags & STRIM_FLAG_NOISE_BY_RANK) && topp;
   const bool cand_sorted = no_lse ? topp : (topk || topp);
   const uint64_t pkey = mix64(p.seed, p.position);
-  const int excl_id = vdr ? draft : -1;
+  const int excl_id = vdr && !gq ? draft : -1;  // (a general-q residual may hold the draft)
 
   // ---- unfiltered Gumbel rows: the chunks' two best tokens ------------------------
   // (and a chunk's near ties of its second best, as its candidates; flag 8: a chunk had
@@ -607,6 +630,73 @@ __device__ __forceinline__ ExactReq finalize_row(const Args& a, int r, int b, in
 
   // ---- phase 3d: draw -----------------------------------------------------------
   int token;
+  if (gq) {
+    // The residual (p - q)^+ of a filtered general-q draft row is zero outside the kept
+    // prefix, so q is looked up for the kept candidates alone (a bitmap word, a rank word
+    // and the draft logit each, one candidate a lane at the usual top-k) and the row ends
+    // here. It went to k_final's streaming resolution, six passes of one workgroup over the
+    // row: V = 151,936, B = 4, k = 3, Vd = 32,768, top-k 20, top-p 0.95 took 587 us a
+    // round, and takes 26.9 us with the lookups.
+    auto qprob = [&](int q) { return q < k1 ? xq_prob(xq, (int)(uint32_t)keys[q]) : 0.0; };
+    const double q0 = qprob(p0);
+    if (a.noise_mode == STRIM_NOISE_ICDF) {
+      auto resid = [&](int q) {
+        const double x = (q == p0 ? w0 : weight(q)) - (q == p0 ? q0 : qprob(q)) * S_kept;
+        return x > 0.0 ? x : 0.0;
+      };
+      double lr = 0.0;
+      for (int q = p0; q < k1; ++q) lr += resid(q);
+      double R;
+      double run = wave_excl_scan_f64(lr, &R);
+      const double tgt = (double)u_draw * R;
+      // the first token whose inclusive residual mass exceeds the target; rounding may push
+      // the target past the end: then the last token with a residual. None has one: the
+      // first kept token
+      int best = n_keep, lastp = -1;
+      for (int q = p0; q < k1; ++q) {
+        const double x = resid(q);
+        if (x > 0.0) {
+          lastp = q;
+          if (best == n_keep && run + x > tgt) best = q;
+        }
+        run += x;
+      }
+      int bp = wave_min_i(best);
+      lastp = wave_max_i(lastp);
+      if (bp >= n_keep) bp = lastp < 0 ? 0 : lastp;
+      token = (int)(uint32_t)keys[bp];
+    } else {
+      const double lse = log(S_kept);
+      double bsc = -INFINITY;
+      uint64_t btk = ~0ull;
+      int bid = -1;
+      for (int q = p0; q < k1; ++q) {
+        const uint64_t key = keys[q];
+        const int id = (int)(uint32_t)key;
+        double base = ((double)fkey_desc_inv((uint32_t)(key >> 32)) - (double)m) - lse;
+        const double qq = q == p0 ? q0 : qprob(q);
+        if (qq != 0.0) {
+          // residual score: log(p - q), excluded where p <= q
+          const double rr = exp(base) - qq;
+          if (!(rr > 0.0)) continue;
+          base = log(rr);
+        }
+        const float u = a.noise ? a.noise[(int64_t)r * a.noise_stride + id]
+                                : philox_uniform(pkey, (uint64_t)id);
+        const double sc = base + gumbel64(u);
+        const uint64_t tk = cand_sorted ? key : (uint64_t)id;
+        if (bid < 0 || sc > bsc || (sc == bsc && tk < btk)) { bsc = sc; btk = tk; bid = id; }
+      }
+      token = wave_argmax_score(bsc, btk, bid);
+      if (token < 0) token = (int)(uint32_t)keys[0];  // p <= q everywhere
+    }
+    // accept iff u < p(d) / q(d)
+    const double qd = xq_prob(xq, draft);
+    const double pd = w_d / S_kept;
+    const double ratio = qd > 0.0 ? pd / qd : (pd > 0.0 ? INFINITY : 0.0);
+    finish_row(a, r, STRIM_OK, token, (double)u_acc < ratio ? 1 : 0, S_kept, m, last_key, PH_DONE);
+    return done;
+  }
   if (a.noise_mode == STRIM_NOISE_ICDF) {
     const double tgt = (double)u_draw * (S_kept - w_d);
     int best = n_keep;
@@ -662,6 +752,9 @@ __device__ __forceinline__ ExactReq finalize_row(const Args& a, int r, int b, in
 // chunk's results visible; an in-kernel device-scope release per workgroup costs far
 // more on gfx950 than the second launch)
 // ---------------------------------------------------------------------------------
+// GQ: a general-q verify (the draft distribution's code: 60 more registers, which cost
+// every other call's rows 0.4 us and the exact resolution 12 %).
+template <bool GQ>
 __global__ __launch_bounds__(FTPB) void k_finalize(Args a) {
   __shared__ FinalShared S;
   // the launch fields of the prefetch, read together (see k_stream)
@@ -674,15 +767,17 @@ __global__ __launch_bounds__(FTPB) void k_finalize(Args a) {
   const RowPre pf = prefetch_row(a, r, b, j);
   const RowParams p = load_params(a, b, j);
   // the general rows are k_gfinal's
-  if (gfinal_row(a.p[b], a.V, a.noise_mode, a.dlog != nullptr && a.verify && j < a.k)) return;
-  const ExactReq q = finalize_row(a, r, b, j, p, pf, S);
+  if (gfinal_row(a.p[b], a.V, a.noise_mode, GQ && j < a.k)) return;
+  const ExactReq q = finalize_row<GQ>(a, r, b, j, p, pf, S);
   // one call site for the exact resolution (an out-of-line call), reached by every
   // thread of a row that needs it
-  if (q.need) finalize_exact(a, r, b, j, p, q.m, q.arg, q.draft, a.verify && j < a.k, q.l_draft, S);
+  if (q.need) finalize_exact<GQ>(a, r, b, j, p, q.m, q.arg, q.draft, a.verify && j < a.k, q.l_draft, S);
 }
 
 hipError_t launch_finalize(const Args& a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
-  return launch_args((const void*)k_finalize, dim3((unsigned)a.R), dim3(FTPB), a, st, e0, e1);
+  const bool gq = a.verify && a.dlog != nullptr;
+  return launch_args(gq ? (const void*)k_finalize<true> : (const void*)k_finalize<false>,
+                     dim3((unsigned)a.R), dim3(FTPB), a, st, e0, e1);
 }
 
 }  // namespace strim

@@ -49,9 +49,9 @@ constexpr float MINP_FAST = 3.3546262e-4f;  // e^-8: min-p at or above bounds ca
 
 enum RowClass : int32_t { CLS_GREEDY = 0, CLS_FAST = 1, CLS_GENERAL = 2, CLS_INVALID = 3 };
 
-// Set by k_finalize and k_gfinal: DONE rows are decided; EXACT rows (filtered general-q
-// verify rows) go to k_final's exact streaming resolution, whose workgroups are four
-// times wider than k_finalize's; QRES rows (unfiltered general-q verify rows) are decided
+// Set by k_finalize and k_gfinal: DONE rows are decided; EXACT rows (general-q
+// verify rows with a filter that bounds no candidates: top-p alone, say) go to k_final's
+// exact streaming resolution, whose workgroups are four times wider than k_finalize's; QRES rows (unfiltered general-q verify rows) are decided
 // by the grid-wide residual draw (qres_kernels.hip), which demotes an icdf row to EXACT
 // when its bucket overflows.
 enum RowPhase : int32_t { PH_DONE = 1, PH_EXACT = 2, PH_QRES = 3 };

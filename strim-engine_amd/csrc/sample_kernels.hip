@@ -6,8 +6,8 @@
 namespace strim {
 
 // ---------------------------------------------------------------------------------
-// k_final: the general-q verify rows k_finalize left in phase EXACT (a filter, or an icdf
-// residual bin too wide for the grid-wide draw), on the exact streaming resolution with
+// k_final: the general-q verify rows k_finalize left in phase EXACT (a filter of the general
+// class, or an icdf residual bin too wide for the grid-wide draw), on the exact streaming resolution with
 // the draft distribution q; every other row is already decided.
 // ---------------------------------------------------------------------------------
 __global__ __launch_bounds__(FIN_T) void k_final(Args a) {

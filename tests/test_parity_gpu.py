@@ -574,6 +574,37 @@ def test_verify_general_q_table_errors(ctx):
     assert (g["accepted"] == 0).all() and (g["token"] == -1).all()
 
 
+@pytest.mark.parametrize("tk,tp,mp,ties", [(1, 1.0, 0.0, False), (2, 0.5, 0.0, False),
+                                           (64, 0.95, 0.0, False), (65, 1.0, 0.0, True),
+                                           (256, 0.99, 0.001, False), (0, 1.0, 0.01, False),
+                                           (0, 0.9, 0.0005, False)])
+@pytest.mark.parametrize("V,grid", [(300, 0.0), (9001, 0.0), (20000, 0.25), (20000, 4.0)])
+def test_verify_general_q_filtered(ctx, tk, tp, mp, ties, V, grid):
+    """Filtered general-q draft rows that k_finalize decides from the row's candidates: kept
+    sets at the edges of a wave (64 / 65), the largest top-k, min-p alone (unsorted kept
+    sets), kept ties; logits rounded to a coarse grid give crowded values (0.25) and tie
+    blocks that overflow the candidate regions (4.0: the exact resolution)."""
+    rng = np.random.default_rng(1000 + tk + V)
+    B, k, Vd = 3, 2, V // 3
+    table = np.sort(rng.choice(V, size=Vd, replace=False)).astype(np.int32)
+    tgt = rng.normal(0, 2.5, size=(B, k + 1, V)).astype(np.float32)
+    if grid:
+        tgt = (np.round(tgt / grid) * grid).astype(np.float32)
+    dl = (0.8 * tgt[:, :k, :][:, :, table]
+          + rng.normal(0, 1.0, size=(B, k, Vd))).astype(np.float32)
+    # drafts among the likeliest (kept: accepted or not) and at random (mostly dropped)
+    top = table[np.argsort(-dl, axis=-1)[:, :, :3]]
+    drafts = top[np.arange(B)[:, None], np.arange(k)[None, :], rng.integers(0, 3, (B, k))]
+    drafts[B - 1] = rng.choice(table, size=k)
+    p = O.make_params(B, temperature=np.array([0.7, 1.0, 0.6]), top_k=tk, top_p=tp, min_p=mp,
+                      flags=O.FLAG_TOPK_KEEP_TIES if ties else 0,
+                      seed=rng.integers(0, 2**63, size=B, dtype=np.uint64), position=5)
+    for mode, rows in ((O.NOISE_ICDF, True), (O.NOISE_GUMBEL, True), (O.NOISE_GUMBEL, False)):
+        say(f"verify general-q filtered k={tk} p={tp} mp={mp} V={V} grid={grid} mode={mode}")
+        check_verify(ctx, tgt, k, drafts.astype(np.int32), p, "bf16", noise_mode=mode,
+                     draft_logits=dl, table=table, label="general-q filtered", row_outputs=rows)
+
+
 # ------------------------------------------------------------------ aux ops ----
 def test_mask_logits(ctx):
     rng = np.random.default_rng(6)
