@@ -23,32 +23,116 @@ __global__ __launch_bounds__(256) void k_mask_logits(const void* logits, int dty
 
 // MTP.nextTokenIndex (Sources/StrimCore/MTP.swift:104-111): argMax over the truncated
 // draft vocab (first max), then the draft->full index table.
-__global__ __launch_bounds__(256) void k_draft_argmax(const void* logits, int dtype, int Vd,
-                                                      int64_t row_stride, const int32_t* table,
-                                                      int32_t* out) {
-  __shared__ float s_v[256 / WAVE];
-  __shared__ int s_i[256 / WAVE];
-  const int r = blockIdx.x;
+//
+// One 1024-thread workgroup per row: a row is at most a few hundred KB, so its time is
+// the memory round trip and the reduction, and a merge across workgroups would cost a
+// second launch. A thread takes its batch's 16-byte loads in flight (32 tokens; the whole of a
+// 32,768-token row in one batch for either dtype). At R = 4, Vd = 32,768 bf16 the kernel
+// takes 4.2 us against 27.7 us with 256 threads of 2-byte loads, one in flight.
+// VEC: rows 16-byte aligned; other rows load token by token, in batches as wide.
+constexpr int DA_T = 1024, DA_N = 32;  // threads, tokens a thread and batch
+template <bool BF16, bool VEC>
+__global__ __launch_bounds__(DA_T) void k_draft_argmax(const void* logits, int Vd,
+                                                       int64_t row_stride, const int32_t* table,
+                                                       int32_t* out) {
+  __shared__ float s_v[DA_T / WAVE];
+  __shared__ int s_i[DA_T / WAVE];
+  const int r = blockIdx.x, t = threadIdx.x, lane = t & (WAVE - 1), w = wave_id();
+  const uint16_t* xb = (const uint16_t*)logits + (int64_t)r * row_stride;
+  const float* xf = (const float*)logits + (int64_t)r * row_stride;
+  auto scalar = [&](int i) { return BF16 ? bf16_to_f32(xb[i]) : xf[i]; };
+  constexpr int E = BF16 ? 8 : 4, U = DA_N / E;  // tokens a load, loads a batch
   float bv = -INFINITY;
   int bi = -1;
-  for (int i = threadIdx.x; i < Vd; i += 256) {
-    const int64_t src = (int64_t)r * row_stride + i;
-    const float x = dtype == STRIM_DTYPE_BF16 ? bf16_to_f32(((const uint16_t*)logits)[src])
-                                              : ((const float*)logits)[src];
-    // NaN never wins; -inf rows fall back to index 0 like argMax over all -inf
-    if (!isnan(x)) argmax_merge(bv, bi, x, i);
+  // (a thread's ids rise: a strict compare keeps the first of equal values; NaN never wins)
+  auto take = [&](float x, int i) {
+    const bool up = x > bv;
+    bv = up ? x : bv;
+    bi = up ? i : bi;
+  };
+  for (int i0 = 0; i0 < Vd; i0 += DA_T * DA_N) {
+    if constexpr (VEC) {
+      // load u of thread t: tokens i0 + (u DA_T + t) E ..; a load that crosses the row end
+      // rereads the row's start and is dropped (the row's last Vd % E tokens: below)
+      uint4 q[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int i = i0 + (u * DA_T + t) * E;
+        const int ic = i + E <= Vd ? i : 0;
+        q[u] = Vd < E ? uint4{0, 0, 0, 0} : BF16 ? *(const uint4*)(xb + ic) : *(const uint4*)(xf + ic);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int i = i0 + (u * DA_T + t) * E;
+        if (i + E > Vd) continue;
+        const uint32_t wd[4] = {q[u].x, q[u].y, q[u].z, q[u].w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if constexpr (BF16) {
+            take(__uint_as_float(wd[e] << 16), i + 2 * e);
+            take(__uint_as_float(wd[e] & 0xFFFF0000u), i + 2 * e + 1);
+          } else {
+            take(__uint_as_float(wd[e]), i + e);
+          }
+        }
+      }
+    } else {
+      float x[DA_N];
+#pragma unroll
+      for (int u = 0; u < DA_N; ++u) {
+        const int i = i0 + u * DA_T + t;
+        x[u] = scalar(i < Vd ? i : 0);
+      }
+#pragma unroll
+      for (int u = 0; u < DA_N; ++u) {
+        const int i = i0 + u * DA_T + t;
+        if (i < Vd) take(x[u], i);
+      }
+    }
   }
-  wave_argmax(bv, bi);
-  if ((threadIdx.x & (WAVE - 1)) == 0) {
-    s_v[threadIdx.x / WAVE] = bv;
-    s_i[threadIdx.x / WAVE] = bi;
+  if (VEC && t < Vd % E) {
+    const int i = Vd / E * E + t;
+    const float x = scalar(i);
+    if (x > bv) take(x, i);
   }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int q = 1; q < 256 / WAVE; ++q) argmax_merge(s_v[0], s_i[0], s_v[q], s_i[q]);
-    int am = s_i[0] < 0 ? 0 : s_i[0];
+  auto block_best = [&]() {
+    wave_argmax(bv, bi);
+    if (lane == 0) {
+      s_v[w] = bv;
+      s_i[w] = bi;
+    }
+    __syncthreads();
+    bv = lane < DA_T / WAVE ? s_v[lane] : -INFINITY;
+    bi = lane < DA_T / WAVE ? s_i[lane] : -1;
+    wave_argmax(bv, bi);
+  };
+  block_best();
+  if (bi < 0) {
+    // no value above -inf: the first that is not NaN, else index 0 (argMax over all -inf)
+    __syncthreads();
+    for (int i = t; i < Vd && bi < 0; i += DA_T)
+      if (!isnan(scalar(i))) bi = i;
+    block_best();
+  }
+  if (t == 0) {
+    const int am = bi < 0 ? 0 : bi;
     out[r] = table ? table[am] : am;
   }
+}
+
+hipError_t launch_draft_argmax(const void* logits, bool bf16, bool vec, int R, int Vd,
+                               int64_t row_stride, const int32_t* table, int32_t* out,
+                               hipStream_t st) {
+  const dim3 grid((unsigned)R), blk(DA_T);
+#define STRIM_DA(B_, V_)                                                                        \
+  hipLaunchKernelGGL((k_draft_argmax<B_, V_>), grid, blk, 0, st, logits, Vd, row_stride, table, \
+                     out)
+  if (bf16 && vec) STRIM_DA(true, true);
+  else if (bf16) STRIM_DA(true, false);
+  else if (vec) STRIM_DA(false, true);
+  else STRIM_DA(false, false);
+#undef STRIM_DA
+  return hipGetLastError();
 }
 
 }  // namespace strim

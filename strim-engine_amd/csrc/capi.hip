@@ -29,8 +29,9 @@ hipError_t launch_qgumbel(const Args& a, bool combine, dim3 grid, hipStream_t st
                           hipEvent_t e1);
 __global__ void k_mask_logits(const void* logits, int dtype, int V, int64_t row_stride,
                               const uint32_t* mask, int64_t mask_stride, float* out);
-__global__ void k_draft_argmax(const void* logits, int dtype, int Vd, int64_t row_stride,
-                               const int32_t* table, int32_t* out);
+hipError_t launch_draft_argmax(const void* logits, bool bf16, bool vec, int R, int Vd,
+                               int64_t row_stride, const int32_t* table, int32_t* out,
+                               hipStream_t st);
 }  // namespace strim
 
 using namespace strim;
@@ -713,9 +714,11 @@ int strim_draft_argmax(void* stream, const void* draft_logits, int32_t dtype, in
                        int32_t* out) {
   if (!draft_logits || !out || !dtype_ok(dtype) || R <= 0 || Vd <= 0 || row_stride < Vd)
     return STRIM_EINVAL;
-  hipLaunchKernelGGL(k_draft_argmax, dim3((unsigned)R), dim3(256), 0, (hipStream_t)stream,
-                     draft_logits, dtype, Vd, row_stride, draft_to_full, out);
-  return launch_status();
+  // (one row: its stride is never used)
+  const bool vec = vec_ok(draft_logits, R > 1 ? row_stride : 0, dtype) != 0;
+  const hipError_t e = launch_draft_argmax(draft_logits, dtype == STRIM_DTYPE_BF16, vec, R, Vd,
+                                           row_stride, draft_to_full, out, (hipStream_t)stream);
+  return e == hipSuccess ? STRIM_OK : STRIM_EHIP;
 }
 
 }  // extern "C"

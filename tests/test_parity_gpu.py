@@ -630,6 +630,38 @@ def test_draft_argmax(ctx):
 
 
 # ------------------------------------------------------------ mirror API ----
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("Vd,stride", [(1, 1), (3, 3), (7, 8), (8, 8), (1001, 1001), (32767, 32768),
+                                       (32768, 32768), (32769, 32784), (70003, 70008)])
+def test_draft_argmax_forms(dtype, Vd, stride):
+    """Rows at the edges of a load and of a batch, aligned and unaligned, with ties (first
+    maximum), NaN (never wins), signed zeros, and rows of -inf and NaN alone."""
+    rng = np.random.default_rng(Vd)
+    x = np.round(rng.normal(0, 2, size=(7, stride))).astype(np.float32)
+    x[1] = -np.inf
+    x[2, : Vd // 2 + 1] = np.nan
+    x[3] = np.nan
+    x[4] = np.where(rng.random(stride) < 0.5, 0.0, -0.0)
+    x[5] = -np.inf
+    x[5, Vd - 1] = -3.0
+    x[6] = np.where(rng.random(stride) < 0.5, np.nan, -np.inf)
+    t = dev_logits(x, dtype)
+    table = np.arange(Vd, dtype=np.int32)[::-1].copy()
+
+    def want(row):
+        ok = ~np.isnan(row)
+        return int(np.flatnonzero(ok & (row == row[ok].max()))[0]) if ok.any() else 0
+
+    ref = np.array([want(row) for row in host_logits(x, dtype)[:, :Vd]])
+    for base in (t[:, :Vd], t.flatten()[1:1 + 6 * stride].view(6, stride)[:, :Vd]):
+        h = base.float().cpu().numpy()
+        exp = ref if base.shape[0] == 7 else np.array([want(row) for row in h])
+        np.testing.assert_array_equal(ops.draft_argmax(base).cpu().numpy(), exp)
+        np.testing.assert_array_equal(ops.draft_argmax(base, dev(table)).cpu().numpy(), table[exp])
+        one = ops.draft_argmax(base[2])
+        assert int(one.item()) == exp[2]
+
+
 def test_sampler_mirror_matches_oracle(ctx):
     from strim_amd.sampler import GenParams, Sampler, SamplingConfig, SpecSampling
 
