@@ -35,7 +35,8 @@ UNITS = [
     # k_gfinal's five leading arguments (the chunk statistics', lattice words' and slots'
     # addresses, the chunk stride and count) arrive preloaded in SGPRs, so its first load
     # is issued before any wait for the argument block
-    ("gfinal_kernels.hip", ["-mllvm", "-amdgpu-kernarg-preload-count=5"]),
+    ("gfinal_kernels.hip", ["-DSTRIM_LW=40", "-mllvm", "-amdgpu-kernarg-preload-count=5"]),
+    ("gfinal_kernels.hip", ["-DSTRIM_LW=64", "-mllvm", "-amdgpu-kernarg-preload-count=5"]),
     ("sample_kernels.hip", []),
     ("qres_kernels.hip", []),
     ("aux_kernels.hip", []),

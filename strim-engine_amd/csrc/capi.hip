@@ -13,6 +13,7 @@
 
 namespace strim {
 hipError_t launch_finalize(const Args& a, hipStream_t st, hipEvent_t e0, hipEvent_t e1);
+template <int LW>
 hipError_t launch_gfinal(const Args& a, hipStream_t st, hipEvent_t e0, hipEvent_t e1);
 hipError_t launch_head(const void* hidden, int64_t hidden_stride, int B, int K,
                        const void* norm_w, float eps, void* xn, const void* W, int64_t w_stride,
@@ -239,7 +240,8 @@ int run_group(strim_ctx* ctx, hipStream_t st, Args& a, int nb, bool probs,
     });
   if (need_gfin)
     timed(ctx, KID_GFINAL, [&](hipEvent_t e0, hipEvent_t e1) {
-      keep(launch_gfinal(a, st, e0, e1));
+      keep(a.W <= LWNARROW ? launch_gfinal<LWNARROW>(a, st, e0, e1)
+                           : launch_gfinal<LWMAX>(a, st, e0, e1));
     });
   if (need_qres) {
     // the residual draw of unfiltered general-q rows (rows in other phases return)

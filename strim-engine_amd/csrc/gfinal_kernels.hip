@@ -16,7 +16,8 @@
 //      order, each token's mass taken from its own l.
 // A zone in a bin that some chunk could not write whole is collected by one streaming
 // pass of this workgroup over the row. A decision below a chunk's window (the lattice
-// cannot place it), rank-indexed noise and rows whose lattice words were not written take
+// cannot place it), rank-indexed noise over more tokens than a zone holds and rows whose
+// lattice words were not written take
 // the exact streaming resolution (exact.hpp).
 //
 // Masses are fixed point, 2^40 per unit of exp(l - m) (RFIX): integer sums make every
@@ -27,8 +28,12 @@
 //
 // One 512-thread workgroup per row. Its time is latency (one global round trip for the
 // chunk statistics and lattice words, then one per zone), so the loads that do not depend
-// on the row's parameters are issued first, and every wave keeps the row's cumulative
-// histogram in its own registers (a decision's bin search needs no barrier).
+// on the row's parameters are issued first, and the leader wave keeps the row's cumulative
+// histogram in its own registers (a decision's bin search needs no barrier). What the
+// leader does not decide alone is out of line (gfinal_rest): with it inline the common
+// path kept 258 scalar values in vector lanes, 11 without (8 constrained rows 20.1 -> 19.6
+// us a call; the wide-nucleus rows 97 -> 92.7, their calls reading the launch's fields by
+// scalar loads instead of copies in scratch memory).
 #include "exact.hpp"
 
 namespace strim {
@@ -41,23 +46,35 @@ constexpr double RFIX = 1099511627776.0;
 constexpr int ZCAP = 4096;                       // keys of one zone
 constexpr int ZQ = ZCAP / GT;                    // zone positions per thread (radix picks)
 constexpr int RADIX_MIN = 256;  // wider zones are picked by radix select, not all pairs
-constexpr int PF = 160;                          // candidates of each chunk prefetched
-// The lattice words and the prefetched candidates are loaded straight into LDS, 1 KB per
-// wave instruction (16 bytes per lane): KW and KP instructions per wave.
-constexpr int LWB = LWMAX * NBW * 8, PFB = LWMAX * PF * 8;  // their bytes
-constexpr int DW = GW - 1;  // the waves that issue them: all but wave 0
-constexpr int KW = (LWB / 1024 + DW - 1) / DW, KP = (PFB / 1024 + DW - 1) / DW;
-static_assert(LWB % 1024 == 0 && PFB % 1024 == 0, "whole 1 KB blocks");
-static_assert(PF <= LCAP && PF % 2 == 0, "prefetch layout");
+constexpr int DW = GW - 1;  // the waves that load into LDS: all but wave 0
+// k_gfinal is built for rows of up to LW = 40 chunks (V <= 163,840) and up to LW = 64
+// (V <= 262,144): the LDS holds every chunk's lattice words, so the wider build keeps
+// fewer prefetched candidates a chunk (PF). Rows past 40 chunks took the exact resolution
+// before: B = 1, V = 248,320, top-p 0.95, rank-indexed Gumbel noise took 586 us a call and
+// takes 26.6. Both are built because a crowded bin's candidates lie past 56 a chunk more
+// often than past 160: the 8-row constrained step of 38 chunks takes 19.6 us, and 25.1 on
+// the wider build.
+template <int LW>
+struct GCfg {
+  static constexpr int PF = LW <= 40 ? 160 : 56;  // candidates of each chunk prefetched
+  // The lattice words and the prefetched candidates are loaded straight into LDS, 1 KB
+  // per wave instruction (16 bytes per lane): KW and KP instructions per wave.
+  static constexpr int LWB = LW * NBW * 8, PFB = LW * PF * 8;  // their bytes
+  static constexpr int KW = (LWB / 1024 + DW - 1) / DW, KP = (PFB / 1024 + DW - 1) / DW;
+  static_assert(LWB % 1024 == 0 && PFB % 1024 == 0, "whole 1 KB blocks");
+  static_assert(PF <= LCAP && PF % 2 == 0, "prefetch layout");
+  static_assert(LW % GW == 0 && LW <= WAVE, "lattice layout");
+};
 constexpr int NOBIN = 1 << 20;                   // "no bin": beyond every window
-static_assert(NBW % WAVE == 0 && LWMAX % GW == 0 && LWMAX <= WAVE, "lattice layout");
+static_assert(NBW % WAVE == 0, "lattice layout");
 static_assert(LCAP <= SLOT && LCAP < 65536, "the candidates fit a chunk's slot region");
 
 // LDS of one k_gfinal workgroup: the two large areas the lattice words and candidates are
 // loaded into (objects of their own: the loads into them are then known not to touch the
 // small state, so reading the chunk statistics does not wait for them), and the rest.
+template <int LW>
 union GBig {
-  uint64_t E[LWMAX * NBW];        // the chunks' lattice words (until they are merged)
+  uint64_t E[LW * NBW];           // the chunks' lattice words (until they are merged)
   struct {                        // a zone: its keys and their masses
     uint64_t zkey[ZCAP];
     uint64_t zmass[ZCAP];
@@ -70,8 +87,9 @@ union GBig {
     XState x;
   } x;
 };
+template <int LW>
 union GPf {
-  Cand pfb[LWMAX * PF];           // each chunk's first PF candidates (prefetched)
+  Cand pfb[LW * GCfg<LW>::PF];         // each chunk's first PF candidates (prefetched)
   uint32_t ccnt[GT * EPT];        // a collect pass: history counts of one window (the
 };                                // prefetched candidates are dropped by then)
 // A step of the decision loop, as the leader wave posts it to the workgroup.
@@ -87,15 +105,16 @@ struct GCmd {
   double thr;
   uint64_t bnd, c0, m0, bmp;
 };
+template <int LW>
 struct GFinalShared {
-  uint16_t pc[LWMAX][NBW];        // per chunk: inclusive count prefix of its window bins
+  uint16_t pc[LW][NBW];           // per chunk: inclusive count prefix of its window bins
   uint32_t rc[NBW];               // row bins: counts
   unsigned long long rm[NBW];     // row bins: masses (RFIX per unit of exp(l - m))
-  int nbch[LWMAX];                // per chunk: window bins written
-  int ncnt[LWMAX];                // per chunk: allowed tokens
-  int dch[LWMAX];                 // per chunk: its top bin's distance below the row's
-  double sch[LWMAX];              // per chunk: its mass sum relative to the row maximum
-  int zoff[LWMAX + 1];            // the Gumbel walk: exclusive offsets of the chunks' parts
+  int nbch[LW];                // per chunk: window bins written
+  int ncnt[LW];                // per chunk: allowed tokens
+  int dch[LW];                 // per chunk: its top bin's distance below the row's
+  double sch[LW];              // per chunk: its mass sum relative to the row maximum
+  int zoff[LW + 1];            // the Gumbel walk: exclusive offsets of the chunks' parts
   float v[GW];
   int i[GW], f[GW];
   double d[GW];
@@ -104,7 +123,7 @@ struct GFinalShared {
   int misc[8];                    // 0 rowfull, 1 rowwin, 2 collect count, 3 some tail
   uint64_t res[2][4];             // a pick: key, count before, mass before, mass (two
   int32_t tag[2];                 // slots, alternating; tag = the pick's number)
-  int zpo[2][LWMAX], zpc[2][LWMAX], zpz[2][LWMAX];  // a zone's parts per chunk: first
+  int zpo[2][LW], zpc[2][LW], zpz[2][LW];  // a zone's parts per chunk: first
                                                     // slot, count, place in the zone
   GCmd cmd;                       // the decision loop's current step
   uint32_t prk[GT];               // a pick: each zone key's rank and the mass before it
@@ -184,7 +203,8 @@ static_assert(LPL == 3, "RowCum holds three bins per lane");
 // the mass before it are summed from R partial counts; the unique key whose interval
 // contains thr writes its result to slot np & 1 (a slot is rewritten two picks later,
 // after every thread has read it). Three barriers.
-__device__ __forceinline__ GHit pick_rank(GFinalShared& S, GBig& G, int np, int z0, int n, bool by_mass,
+template <int LW>
+__device__ __forceinline__ GHit pick_rank(GFinalShared<LW>& S, GBig<LW>& G, int np, int z0, int n, bool by_mass,
                                           double thr, uint64_t bound, int excl, uint64_t cnt0,
                                           uint64_t mass0) {
   const int t = threadIdx.x;
@@ -258,7 +278,8 @@ __device__ __forceinline__ GHit pick_rank(GFinalShared& S, GBig& G, int np, int 
 // (double)before(d) <= thr < (double)(before(d) + weight(d)), as pick_rank's rule for one
 // key. The candidates narrow to d until every bit is fixed: about five passes of three
 // barriers for the keys of one lattice bin.
-__device__ __forceinline__ GHit pick_sorted(GFinalShared& S, GBig& G, int np, int z0, int n,
+template <int LW>
+__device__ __forceinline__ GHit pick_sorted(GFinalShared<LW>& S, GBig<LW>& G, int np, int z0, int n,
                                             bool by_mass, double thr, uint64_t bound, int excl,
                                             uint64_t cnt0, uint64_t mass0) {
   const int t = threadIdx.x, lane = t & (WAVE - 1), w = wave_id();
@@ -395,7 +416,8 @@ __device__ __forceinline__ GHit pick_sorted(GFinalShared& S, GBig& G, int np, in
 
 // Sum of the masses of the zone's keys <= bound, zone zkey/zmass[z0, z0 + n) (every
 // thread; two barriers).
-__device__ __forceinline__ uint64_t zone_mass_upto(GFinalShared& S, GBig& G, int z0, int n,
+template <int LW>
+__device__ __forceinline__ uint64_t zone_mass_upto(GFinalShared<LW>& S, GBig<LW>& G, int z0, int n,
                                                   uint64_t bound) {
   const int t = threadIdx.x, lane = t & (WAVE - 1), w = wave_id();
   uint64_t s = 0ull;
@@ -410,16 +432,38 @@ __device__ __forceinline__ uint64_t zone_mass_upto(GFinalShared& S, GBig& G, int
   return tot;
 }
 
+// The launch's argument block where the hardware put it, for the functions that are not
+// inlined: its address (two registers) is passed, and they read the fields they use by
+// scalar loads. The block, or the streaming passes' view of it, passed by value goes
+// through scratch memory (4 us a call of the cooperative decisions). Such functions are
+// marked not_tail_called: a call the compiler could make a tail call makes the function
+// save every register it may keep for its caller, some hundred scratch stores and loads
+// a lane (10 us).
+struct GKernArgs {  // k_gfinal's arguments as the kernel-argument segment lays them out
+  const ChunkStat* cstat;
+  const unsigned long long* lat;
+  const Cand* slot;
+  int wmax, W;
+  Args a;
+};
+typedef __attribute__((address_space(4))) const Args c_args;
+__device__ __forceinline__ uint64_t kernel_args() {
+  return (uint64_t)(uintptr_t)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(GKernArgs, a);
+}
+__device__ __forceinline__ const Args& args_at(uint64_t p) {
+  return *(const Args*)(c_args*)uniform_copy(p);
+}
 // Out-of-line forms of the rare paths (their code stays out of the common path's
 // instruction stream; the LDS arrives as an address-space-typed pointer, and only the
 // launch fields they read are passed: a reference to the argument block would copy it
 // to private memory).
-__device__ __noinline__ GHit pick_sorted_ool(lds_t<GFinalShared>* Sl, lds_t<GBig>* Gl, int np,
+template <int LW>
+__device__ __noinline__ GHit pick_sorted_ool(lds_t<GFinalShared<LW>>* Sl, lds_t<GBig<LW>>* Gl, int np,
                                              int z0, int n, bool by_mass, double thr,
                                              uint64_t bound, int excl, uint64_t cnt0,
                                              uint64_t mass0) {
-  GFinalShared& S = *(GFinalShared*)Sl;
-  GBig& G = *(GBig*)Gl;
+  GFinalShared<LW>& S = *(GFinalShared<LW>*)Sl;
+  GBig<LW>& G = *(GBig<LW>*)Gl;
   return pick_sorted(S, G, np, z0, n, by_mass, thr, bound, excl, cnt0, mass0);
 }
 // The last key passing min-p, (double)l - (double)m >= lmp: the first fkey (descending l)
@@ -431,12 +475,29 @@ __device__ __noinline__ uint32_t minp_last_fkey(float m, double lmp) {
 }
 // Gumbel over every kept candidate of a row (key <= bound, not the draft): the chunks'
 // candidate entries of bins up to the bound's bin bb, scored in fp64. Returns the token
-// (-1: none kept but the draft).
-__device__ __noinline__ int gumbel_kept(lds_t<GFinalShared>* Sl, const Cand* base,
-                                        const float* noise, int W, int bb, uint64_t bound,
-                                        int draft, const RowParams p, float m, uint64_t S1,
-                                        bool cand_sorted) {
-  GFinalShared& S = *(GFinalShared*)Sl;
+// (-1: none kept but the draft). by_rank: a token's noise is that of its rank in the
+// row's order. The entries are first laid out by row bin (each bin's first place from the
+// row's counts, S.rc, a token's place in its bin by an atomic), and a token's rank is its
+// bin's first place plus the smaller keys of its bin, so a nucleus of a few thousand
+// tokens needs no sort; past ZCAP entries: -2, the exact resolution.
+template <int LW>
+__attribute__((not_tail_called)) __device__ __noinline__ int gumbel_kept(
+    uint64_t kargs, int r, lds_t<GFinalShared<LW>>* Sl, lds_t<GBig<LW>>* Gl, int bb,
+    uint64_t bound, int draft, float m, uint64_t S1) {
+  const Args& a = args_at(kargs);
+  r = __builtin_amdgcn_readfirstlane(r);
+  int b, j;
+  row_bj(a, r, b, j);
+  const RowParams p = load_params(a, b, j);
+  const int W = a.W;
+  const Cand* base = a.s.slot + (int64_t)r * a.s.wmax * SLOT;
+  const float* noise = a.noise ? a.noise + (int64_t)r * a.noise_stride : nullptr;
+  const bool topk = p.top_k > 0 && p.top_k < a.V, topp = p.top_p < 1.0f;
+  const bool cand_sorted = (p.flags & STRIM_FLAG_SCORE_NO_LSE) ? topp : (topk || topp);
+  const bool by_rank = (p.flags & STRIM_FLAG_NOISE_BY_RANK) && topp;
+  GFinalShared<LW>& S = *(GFinalShared<LW>*)Sl;
+  GBig<LW>& G = *(GBig<LW>*)Gl;
+  __syncthreads();  // (the last pick's reads of its state)
   const int t = threadIdx.x, lane = t & (WAVE - 1), w = wave_id();
   if (w == 0) {
     // lane c: chunk c's entries up to its part of the bound's bin
@@ -448,15 +509,32 @@ __device__ __noinline__ int gumbel_kept(lds_t<GFinalShared>* Sl, const Cand* bas
     const int zof = (int)wave_incl_scan_u32((uint32_t)lim) - lim;
     if (lane < W) S.zoff[lane] = zof;
     if (lane == W - 1) S.zoff[W] = zof + lim;
+    if (by_rank) {  // the row bins' counts become their exclusive prefixes
+      uint32_t c[LPL], tot = 0u;
+#pragma unroll
+      for (int q = 0; q < LPL; ++q) {
+        c[q] = S.rc[LPL * lane + q];
+        tot += c[q];
+      }
+      uint32_t run = wave_incl_scan_u32(tot) - tot;
+#pragma unroll
+      for (int q = 0; q < LPL; ++q) {
+        S.rc[LPL * lane + q] = run;
+        run += c[q];
+      }
+    }
   }
+  if (by_rank && t < NBW) S.prk[t] = 0u;
   __syncthreads();
   const int N = S.zoff[W];
+  if (by_rank && N > ZCAP) return -2;
   const bool no_lse = (p.flags & STRIM_FLAG_SCORE_NO_LSE) != 0;
   const double lse = log((double)S1 / RFIX);
   const uint64_t pkey = mix64(p.seed, p.position);
   double bsc = -INFINITY;
   uint64_t btk = ~0ull;
   int bid = -1;
+  const float arow = floorf(m * (float)LBS);
   for (int i = t; i < N; i += GT) {
     // the chunk holding entry i: the last c with zoff[c] <= i
     int lo = 0, hi = W - 1;
@@ -467,6 +545,11 @@ __device__ __noinline__ int gumbel_kept(lds_t<GFinalShared>* Sl, const Cand* bas
     }
     const Cand x = base[(int64_t)lo * SLOT + (i - S.zoff[lo])];
     const uint64_t k = ckey(x.l, x.id);
+    if (by_rank) {  // (every entry: those of the bound's bin past it rank after it)
+      const int bq = row_bin(arow, x.l);
+      G.z.zkey[S.rc[bq] + atomicAdd(&S.prk[bq], 1u)] = k;
+      continue;
+    }
     if (k > bound || x.id == draft) continue;
     const float u = noise ? noise[x.id] : philox_uniform(pkey, (uint64_t)x.id);
     const double bs = no_lse ? (double)x.l : ((double)x.l - (double)m) - lse;
@@ -478,8 +561,50 @@ __device__ __noinline__ int gumbel_kept(lds_t<GFinalShared>* Sl, const Cand* bas
       bid = x.id;
     }
   }
+  if (by_rank) {
+    __syncthreads();
+    for (int i = t; i < N; i += GT) {
+      const uint64_t k = G.z.zkey[i];
+      if (k > bound) continue;
+      const float l = key_l(k);
+      const int bq = row_bin(arow, l);
+      const int z0 = (int)S.rc[bq], z1 = z0 + (int)S.prk[bq];
+      int rank = z0;
+      for (int q = z0; q < z1; ++q) rank += G.z.zkey[q] < k ? 1 : 0;
+      const float u = noise ? noise[rank] : philox_uniform(pkey, (uint64_t)rank);
+      const double sc = (no_lse ? (double)l : ((double)l - (double)m) - lse) + gumbel64(u);
+      if (bid < 0 || sc > bsc || (sc == bsc && k < btk)) {
+        bsc = sc;
+        btk = k;
+        bid = (int)(uint32_t)k;
+      }
+    }
+  }
   block_argmax_score<GT>(bsc, btk, bid, S.d, S.u, S.ii, &S.misc[4]);
   return S.misc[4];
+}
+
+// The streaming passes' view of the launch (collect passes and the exact resolution).
+__device__ __forceinline__ XArgs xargs_of(const Args& a) {
+  XArgs xa;
+  xa.logits = a.logits;
+  xa.row_stride = a.row_stride;
+  xa.dtype = a.dtype;
+  xa.vec_ok = a.vec_ok;
+  xa.V = a.V;
+  xa.H = a.H;
+  xa.verify = a.verify;
+  xa.k = a.k;
+  xa.noise_mode = a.noise_mode;
+  xa.mask = a.mask;
+  xa.mask_stride = a.mask_stride;
+  xa.hist = a.hist;
+  xa.hist_len = a.hist_len;
+  xa.drafts = a.drafts;
+  xa.noise = a.noise;
+  xa.noise_stride = a.noise_stride;
+  xa.has_q = 0;
+  return xa;
 }
 
 // The LDS a collect pass writes (address-space-typed: see lds_t).
@@ -632,15 +757,15 @@ __device__ __forceinline__ float least_x_for(float T, float A) {
 // pass of the workgroup over the row's logits (the chain recomputed per window), into
 // key / mass. Returns their number, -1 past ZCAP. Out of line: the common path of
 // k_gfinal keeps none of the pass's registers.
-__device__ __noinline__ int collect_zone(const XArgs a_in, int r, int b, int j,
-                                         const RowParams p_in, float at, float m,
+__attribute__((not_tail_called)) __device__ __noinline__ int collect_zone(uint64_t kargs, int r, float at, float m,
                                          const ZoneLds z_in) {
-  const XArgs a = uniform_copy(a_in);
-  const RowParams p = uniform_copy(p_in);
+  const Args& ka = args_at(kargs);
+  const XArgs a = xargs_of(ka);
   const ZoneLds z = uniform_copy(z_in);
   r = __builtin_amdgcn_readfirstlane(r);
-  b = __builtin_amdgcn_readfirstlane(b);
-  j = __builtin_amdgcn_readfirstlane(j);
+  int b, j;
+  row_bj(ka, r, b, j);
+  const RowParams p = load_params(ka, b, j);
   // (readfirstlane takes an int: floats go through their bits)
   at = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(at)));
   m = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(m)));
@@ -714,16 +839,367 @@ __device__ __noinline__ int collect_zone(const XArgs a_in, int r, int b, int j,
   return n <= ZCAP ? n : -1;
 }
 
+// The row's totals and limits from the merged lattice (every lane; scalar: see
+// uniform_copy).
+struct GTotals {
+  int rowwin, rowfull, anytail, n_all;
+  uint64_t S0;
+};
+template <int LW>
+__device__ __forceinline__ GTotals row_totals(GFinalShared<LW>& S, int W) {
+  const int lane = threadIdx.x & (WAVE - 1);
+  GTotals o;
+  o.rowwin = uniform_copy(S.misc[1] < NBW ? S.misc[1] : NBW);
+  o.rowfull = uniform_copy(S.misc[0] < o.rowwin ? S.misc[0] : o.rowwin);
+  o.anytail = uniform_copy(S.misc[3]);
+  o.n_all = wave_sum(lane < W ? S.ncnt[lane] : 0);
+  const double S_all = wave_sum(lane < W ? S.sch[lane] : 0.0);
+  o.S0 = (uint64_t)__double2ull_rn(S_all * RFIX);
+  return o;
+}
+// The row's cumulative histogram in the registers of the calling wave, scaled from each
+// bin's lattice unit to RFIX per unit of exp(l - m): scale(b) =
+// 8 exp(arow / LBS - m) 2^(-b log2(e) / LBS).
+template <int LW>
+__device__ __forceinline__ RowCum row_cum(GFinalShared<LW>& S, float arow, float m) {
+  const int lane = threadIdx.x & (WAVE - 1);
+  RowCum rcum;
+  const float base = 8.0f * expf(arow * (1.0f / (float)LBS) - m);
+  uint32_t lc = 0u;
+  uint64_t lm = 0ull;
+#pragma unroll
+  for (int q = 0; q < LPL; ++q) {
+    const int bq = LPL * lane + q;
+    rcum.cq(q) = S.rc[bq];
+    const float sc = base * __builtin_amdgcn_exp2f(-(float)bq * (1.44269504f / (float)LBS));
+    rcum.mq(q) = (uint64_t)__double2ull_rn((double)S.rm[bq] * (double)sc);
+    lc += rcum.cq(q);
+    lm += rcum.mq(q);
+  }
+  uint32_t bc = wave_incl_scan_u32(lc) - lc;
+  uint64_t bm = wave_incl_scan_u64(lm) - lm;
+#pragma unroll
+  for (int q = 0; q < LPL; ++q) {
+    bc += rcum.cq(q);
+    bm += rcum.mq(q);
+    rcum.cq(q) = bc;
+    rcum.mq(q) = bm;
+  }
+  return rcum;
+}
+
+// What the cooperative decisions and the exact resolution need of a row.
+struct GRow {
+  float m, l_draft, u_draw, u_acc;
+  int arg, draft, exact;
+};
+
+// The rows the leader wave does not decide alone: the cooperative decisions (from the
+// merged lattice in S), and the exact resolution where they fail (or g.exact). Out of
+// line, all of it: the common path keeps none of its registers.
+template <int LW>
+__attribute__((not_tail_called)) __device__ __noinline__ XOut gfinal_rest(uint64_t kargs, int r, const GRow g_in,
+                                         lds_t<GFinalShared<LW>>* Sl, lds_t<GBig<LW>>* Gl,
+                                         lds_t<GPf<LW>>* Pl) {
+  constexpr int PF = GCfg<LW>::PF;
+  const GRow g0 = uniform_copy(g_in);
+  const Args& a = args_at(kargs);
+  r = __builtin_amdgcn_readfirstlane(r);
+  int b, j;
+  row_bj(a, r, b, j);
+  const RowParams p = load_params(a, b, j);
+  GFinalShared<LW>& S = *(GFinalShared<LW>*)Sl;
+  GBig<LW>& G = *(GBig<LW>*)Gl;
+  GPf<LW>& P = *(GPf<LW>*)Pl;
+  const int t = threadIdx.x, lane = t & (WAVE - 1), w = wave_id();
+  const int V = a.V, W = a.W, arg = g0.arg, draft = g0.draft;
+  const float m = g0.m, l_draft = g0.l_draft, u_draw = g0.u_draw, u_acc = g0.u_acc;
+  const bool vdr = a.verify && j < a.k;
+  const Cand* slots = a.s.slot + (int64_t)r * a.s.wmax * SLOT;
+  const float arow = floorf(m * (float)LBS);
+  XOut out{STRIM_OK, -1, 0, 0.0, 0ull};
+  auto decide = [&]() -> bool {
+    const GTotals tt = row_totals<LW>(S, W);
+    RowCum rcum;
+    if (w == 0) rcum = row_cum<LW>(S, arow, m);
+    const int rowwin = tt.rowwin, rowfull = tt.rowfull, n_all = tt.n_all;
+    const bool anytail = tt.anytail != 0;
+    const uint64_t S0 = tt.S0;
+    const bool topk = p.top_k > 0 && p.top_k < V;
+    const bool topp = p.top_p < 1.0f;
+    const bool minp = p.min_p > 0.0f;
+    const bool icdf = a.noise_mode == STRIM_NOISE_ICDF;
+    bool pfok = true;  // the prefetched candidates are in LDS
+    // The zone in LDS: up to two bins, zb[h] at [zo[h], zo[h] + zn[h]). A chunk's part of a
+    // bin comes from its prefetched candidates when it lies among them, else from its slot
+    // region; a bin some chunk could not write whole is collected by a streaming pass.
+    int zb[2] = {-1, -1}, zo[2] = {0, 0}, zn[2] = {0, 0}, npick = 0;
+
+    // The decisions, in order, through one loop (its code is fetched once):
+    //   0 top-k: the k-th key in order (every key counts);
+    //   1 min-p: the kept mass of the keys whose l passes, (double)l - (double)m >= lmp;
+    //   2 top-p: the last kept token is the first whose inclusive mass exceeds P Sk (a
+    //     token is dropped iff the mass before it exceeds P, SpecSampling.swift:62-66);
+    //   3 the icdf draw over the kept keys without the draft.
+    // The leader finds each step's bin and lays out its zone; every wave then loads the
+    // zone and takes part in the pick, and keeps the same state (all of it uniform).
+    // The kept set before top-p: keys <= bound, mass Sk, the bound's bin bbin (NOBIN:
+    // none inside the window); after it: bound1, S1, bb1.
+    uint64_t bound = ~0ull, Sk = S0, bound1 = ~0ull, S1 = S0, wd = 0ull;
+    int bbin = NOBIN, bb1 = NOBIN, xb = NOBIN, token = -1;
+    for (int step = 0; step < 4; ++step) {
+      if (step == 0 && !topk) continue;
+      if (step == 1 && !minp) continue;
+      if (step == 2) {
+        bound1 = bound;
+        S1 = Sk;
+        bb1 = bbin;
+        if (!topp) continue;
+      }
+      if (step == 3) {
+        // the draft of a verify row: kept? its mass and bin
+        if (vdr && l_draft > -INFINITY && ckey(l_draft, draft) <= bound1) {
+          wd = rmass(l_draft, m);
+          xb = row_bin(arow, l_draft);
+        }
+        if (!icdf) break;
+        if (S1 <= wd) {
+          token = arg;  // only the draft kept: the first kept token
+          break;
+        }
+      }
+      // ---- the leader: this step's bin and zone -------------------------------------
+      if (w == 0) {
+        GCmd cmd;
+        cmd.op = GOP_PICK;
+        cmd.load = 0;
+        cmd.also = -1;
+        cmd.by_mass = 1;
+        cmd.excl = -1;
+        cmd.thr = 0.0;
+        cmd.bnd = ~0ull;
+        cmd.bmp = ~0ull;
+        int bz = -1, bfall = NOBIN;
+        uint64_t xw = 0ull;
+        int xbn = NOBIN;
+        if (step == 0) {
+          if (n_all < p.top_k) cmd.op = GOP_SKIP;  // every allowed token is kept
+          cmd.by_mass = 0;
+          cmd.thr = (double)(p.top_k - 1);
+        } else if (step == 1) {
+          const uint32_t flast = minp_last_fkey(m, p.lmp);
+          cmd.bmp = ((uint64_t)flast << 32) | 0xFFFFFFFFull;
+          cmd.op = GOP_SUM;
+          if (cmd.bmp >= bound) {
+            cmd.op = GOP_SKIP;
+          } else {
+            bz = row_bin(arow, fkey_desc_inv(flast));
+            // below the window: with no token below some chunk's window every allowed
+            // token passes (the bound alone is set), else the lattice cannot tell
+            if (bz >= rowwin) cmd.op = anytail ? GOP_FAIL : GOP_BOUND;
+          }
+        } else if (step == 2) {
+          cmd.thr = (double)p.top_p * (double)Sk;
+          cmd.bnd = bound;
+          bfall = bbin;  // the cut lies in the bound's bin when no bin above it crosses
+        } else {
+          cmd.thr = (double)u_draw * (double)(S1 - wd);
+          cmd.bnd = bound1;
+          cmd.excl = draft;
+          xw = wd;
+          xbn = xb;
+          bfall = bb1;
+        }
+        if (cmd.op == GOP_PICK || cmd.op == GOP_SUM) {
+          if (bz < 0) {
+            const int lim = bfall < rowwin ? bfall : rowwin;
+            bz = rcum.find(cmd.by_mass, cmd.thr, lim, xw, xbn);
+            if (bz >= lim) bz = bfall < rowwin ? bfall : NOBIN;
+            // top-p of a sample row: the icdf draw's bin, when it can be told now, is
+            // loaded with the cut's (the kept mass lies between the masses before and
+            // through the cut's bin, so the draw's threshold lies between u times each)
+            if (bz < NOBIN && step == 2 && icdf && !vdr) {
+              const int blo = rcum.find(true, (double)u_draw * (double)rcum.mass(bz - 1), bz + 1, 0ull, NOBIN);
+              const int bhi = rcum.find(true, (double)u_draw * (double)rcum.mass(bz), bz + 1, 0ull, NOBIN);
+              if (blo == bhi && blo <= bz) cmd.also = blo;
+            }
+          }
+          if (bz >= rowwin) {
+            cmd.op = GOP_FAIL;
+          } else if (zb[0] != bz && zb[1] != bz) {
+            if (bz >= rowfull) {
+              cmd.load = 2;
+              cmd.also = -1;
+            } else {
+              const uint64_t cr = rcum.cnt(bz) - rcum.cnt(bz - 1);
+              const int also = cmd.also;
+              const bool two = also >= 0 && also != bz && also < rowfull &&
+                               cr + rcum.cnt(also) - rcum.cnt(also - 1) <= (uint64_t)GT;
+              cmd.also = two ? also : -1;
+              if (cr > (uint64_t)ZCAP) cmd.op = GOP_FAIL;
+              // lane c: chunk c's parts of the bins and their places in the zone
+              const int bins[2] = {bz, cmd.also};
+              int n[2];
+#pragma unroll
+              for (int hh = 0; hh < 2; ++hh) {
+                int cnt = 0, off = 0;
+                if (lane < W && bins[hh] >= 0) {
+                  const int lb = bins[hh] - S.dch[lane];
+                  if (lb >= 0 && lb < S.nbch[lane]) {
+                    off = lb > 0 ? (int)S.pc[lane][lb - 1] : 0;
+                    cnt = (int)S.pc[lane][lb] - off;
+                  }
+                }
+                const int zo_ = (int)wave_incl_scan_u32((uint32_t)cnt) - cnt;
+                n[hh] = __builtin_amdgcn_readlane(zo_ + cnt, WAVE - 1);
+                if (lane < W) {
+                  S.zpo[hh][lane] = off;
+                  S.zpc[hh][lane] = cnt;
+                  S.zpz[hh][lane] = zo_ + (hh ? n[0] : 0);
+                }
+              }
+              cmd.load = 1;
+              cmd.n0 = n[0];
+              cmd.n1 = n[1];
+            }
+          }
+          cmd.c0 = rcum.cnt(bz - 1);
+          cmd.m0 = rcum.mass(bz - 1) - (bz - 1 >= xbn ? xw : 0ull);
+        }
+        cmd.bz = bz;
+        if (lane == 0) S.cmd = cmd;
+      }
+      __syncthreads();
+      const GCmd cmd = uniform_copy(S.cmd);
+      if (cmd.op == GOP_FAIL) return false;
+      if (cmd.op == GOP_SKIP) continue;
+      if (cmd.op == GOP_BOUND) {
+        bound = cmd.bmp;
+        continue;
+      }
+      const int bz = cmd.bz;
+      // ---- every wave: the zone ------------------------------------------------------
+      if (cmd.load == 1) {
+        // wave w copies the parts of chunks w, w + GW, ...: from the prefetched
+        // candidates where they lie among them, else from the chunk's slot region
+        for (int cq = w; cq < W; cq += GW) {
+#pragma unroll
+          for (int hh = 0; hh < 2; ++hh) {
+            const int o = S.zpo[hh][cq], cn = S.zpc[hh][cq], z0 = S.zpz[hh][cq];
+            for (int i = lane; i < cn; i += WAVE) {
+              const int e = o + i;
+              Cand x;  // (two branches: one pointer to either memory would make flat loads)
+              if (pfok && e < PF) {
+                const lds_t<Cand>& y = ((const lds_t<Cand>*)P.pfb)[cq * PF + e];
+                x = Cand{y.l, y.id};
+              } else {
+                const glb_t<const Cand>& y = ((const glb_t<const Cand>*)slots)[(int64_t)cq * SLOT + e];
+                x = Cand{y.l, y.id};
+              }
+              if (z0 + i < ZCAP) {
+                G.z.zkey[z0 + i] = ckey(x.l, x.id);
+                G.z.zmass[z0 + i] = rmass(x.l, m);
+              }
+            }
+          }
+        }
+        __syncthreads();
+        zb[0] = bz;
+        zo[0] = 0;
+        zn[0] = cmd.n0;
+        zb[1] = cmd.also;
+        zo[1] = cmd.n0;
+        zn[1] = cmd.n1;
+      } else if (cmd.load == 2) {
+        const int n = collect_zone(kargs, r, arow - (float)bz, m,
+                                   ZoneLds{(lds_t<uint64_t>*)G.z.zkey, (lds_t<uint64_t>*)G.z.zmass,
+                                           (lds_t<uint32_t>*)P.ccnt, (lds_t<int>*)&S.misc[2]});
+        pfok = false;  // (the pass's history counts took the prefetched candidates' LDS)
+        if (n < 0) return false;
+        zb[0] = bz;
+        zo[0] = 0;
+        zn[0] = n;
+        zb[1] = -1;
+      }
+      const int h = zb[0] == bz ? 0 : 1;
+      if (cmd.op == GOP_SUM) {
+        // min-p: the kept mass is everything before the bound's bin and the zone's keys
+        // up to the bound
+        bound = cmd.bmp;
+        Sk = cmd.m0 + zone_mass_upto(S, G, zo[h], zn[h], bound);
+        bbin = bz;
+        continue;
+      }
+      // ---- the pick: the key whose cumulative interval contains thr ------------------
+      GHit g;
+      {
+        const int np = npick++;
+        if (zn[h] <= RADIX_MIN)
+          g = pick_rank(S, G, np, zo[h], zn[h], cmd.by_mass != 0, cmd.thr, cmd.bnd, cmd.excl,
+                        cmd.c0, cmd.m0);
+        else
+          g = pick_sorted_ool(Sl, Gl, np, zo[h], zn[h], cmd.by_mass != 0, cmd.thr, cmd.bnd,
+                              cmd.excl, cmd.c0, cmd.m0);
+      }
+      if (step == 0) {
+        if (g.key == ~0ull) return false;
+        if (p.flags & STRIM_FLAG_TOPK_KEEP_TIES) {
+          // the keys tied with the k-th one are kept too (same value, same bin)
+          bound = g.key | 0xFFFFFFFFull;
+          Sk = cmd.m0 + zone_mass_upto(S, G, zo[h], zn[h], bound);
+        } else {
+          bound = g.key;
+          Sk = g.mass_before + g.mass;
+        }
+        bbin = bz;
+      } else if (step == 2) {
+        if (g.key != ~0ull) {
+          bound1 = g.key;
+          S1 = g.mass_before + g.mass;
+          bb1 = bz;
+        } else if (bz != bbin) {
+          return false;
+        }
+      } else {
+        if (g.key == ~0ull) return false;
+        token = (int)(uint32_t)g.key;
+      }
+    }
+    if (!icdf) {
+      // Gumbel: every kept candidate (key <= bound1, not the draft)
+      if (bb1 >= rowfull) return false;  // every kept token must be a candidate
+      token = gumbel_kept<LW>(kargs, r, Sl, Gl, bb1, bound1, draft, m, S1);
+      if (token == -2) return false;
+      if (token < 0) token = arg;  // only the draft kept
+    }
+    out.accept = vdr && ((double)u_acc < (double)wd / (double)S1) ? 1 : 0;
+    out.token = token;
+    out.sig = (double)S1 / RFIX;
+    out.last_key = bound1;
+    return true;
+  };
+  if (!g0.exact && decide()) return out;
+
+  // ---- the exact streaming resolution ----------------------------------------------
+  const XScratch xs = xscratch(G.x.xkey, G.x.xhc, G.x.xcnt, G.x.xu2, S.d, S.u, S.ii);
+  __builtin_amdgcn_s_waitcnt(0);  // (its LDS overlaps the lattice words' and candidates')
+  __syncthreads();
+  return exact_row<GT, false>(xargs_of(a), r, b, j, p, m, arg, draft, vdr, l_draft, xs,
+                              *(lds_t<XState>*)&G.x.x);
+}
+
 // The leading arguments repeat fields of `a` (a.s.cstat, a.s.lat, a.s.slot, a.s.wmax,
 // a.W): built with kernel-argument preloading, they arrive in SGPRs, so the chunk
 // statistics' load is issued before any wait for the argument block.
+template <int LW>
 __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
                                                 const unsigned long long* pre_lat,
                                                 const Cand* pre_slot, int pre_wmax, int pre_W,
                                                 Args a) {
-  __shared__ GFinalShared S;
-  __shared__ GBig G;
-  __shared__ GPf P;
+  constexpr int PF = GCfg<LW>::PF, KW = GCfg<LW>::KW, KP = GCfg<LW>::KP;
+  __shared__ GFinalShared<LW> S;
+  __shared__ GBig<LW> G;
+  __shared__ GPf<LW> P;
   // the chunk statistics first, their address from the preloaded arguments alone (a row
   // of at most 64 chunks: every wave loads all of them, lane c chunk c; wider rows:
   // thread t chunk t)
@@ -758,7 +1234,7 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
   const unsigned long long* lwp = pre_lat + (int64_t)r * pre_wmax * NBW;
   const Cand* slots = pre_slot + (int64_t)r * pre_wmax * SLOT;
   if (w > 0) {
-    const int wl = W <= LWMAX ? W : 1;
+    const int wl = W <= LW ? W : 1;
     const int nwb = (wl * NBW * 8 + 1023) / 1024, npb = (wl * PF * 8 + 1023) / 1024;
 #pragma unroll
     for (int q = 0; q < KW; ++q) {
@@ -852,34 +1328,15 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
     u_draw = pu_draw;
     u_acc = pu_acc;
   }
-  // the streaming passes' view of the launch (collect passes and the exact resolution)
-  XArgs xa;
-  xa.logits = a.logits;
-  xa.row_stride = a.row_stride;
-  xa.dtype = a.dtype;
-  xa.vec_ok = a.vec_ok;
-  xa.V = a.V;
-  xa.H = a.H;
-  xa.verify = a.verify;
-  xa.k = a.k;
-  xa.noise_mode = a.noise_mode;
-  xa.mask = a.mask;
-  xa.mask_stride = a.mask_stride;
-  xa.hist = a.hist;
-  xa.hist_len = a.hist_len;
-  xa.drafts = a.drafts;
-  xa.noise = a.noise;
-  xa.noise_stride = a.noise_stride;
-  xa.has_q = 0;
 
   // ---- the row's lattice ---------------------------------------------------------
   const float arow = floorf(m * (float)LBS);
-  const bool lat = W <= LWMAX && !(flags & 8) && fabsf(arow) < 0x1p+23f;
-  auto decide = [&]() -> bool {
+  const bool lat = W <= LW && !(flags & 8) && fabsf(arow) < 0x1p+23f;
+  auto decide = [&]() -> int {  // solo's verdict
     // per chunk (the thread of chunk t): its distance below the row's top bin, its mass
     // sum relative to the row maximum, how far down its bins are whole; the chunks'
     // lattice words staged in LDS with their count prefixes (for the gathers)
-    // (the chunks' threads are all in wave 0, W <= LWMAX: the row's limits are wave
+    // (the chunks' threads are all in wave 0, W <= LW: the row's limits are wave
     // reductions there, one store each; an LDS atomic from every lane to one word is
     // serialised lane by lane, about 2.5 us for 38 chunks)
     if (t < NBW) {
@@ -921,19 +1378,19 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     // every row bin: the counts and masses of its chunks' bins. Wave w takes chunks w,
-    // w + 8, ... (at most LWMAX / 8), lane l row bins 3 l .. 3 l + 2 of each (a chunk's
+    // w + 8, ... (at most LW / 8), lane l row bins 3 l .. 3 l + 2 of each (a chunk's
     // bins read with the one before them: four words for three bins, all requested
     // before any is used); a lattice bin's masses share their unit, so they add as
     // integers, and each row bin gets one LDS atomic per wave. Each chunk's inclusive
     // count prefixes are kept for the gathers.
     {
-      static_assert(LPL == 3 && LWMAX % GW == 0, "three row bins a lane, whole chunk rounds");
+      static_assert(LPL == 3 && LW % GW == 0, "three row bins a lane, whole chunk rounds");
       const int dreg = lane < W ? S.dch[lane] : NOBIN;
       const int nbreg = lane < W ? S.nbch[lane] : 0;
       uint32_t cq[LPL] = {0u, 0u, 0u};
       uint64_t mq[LPL] = {0ull, 0ull, 0ull};
 #pragma unroll
-      for (int k = 0; k < LWMAX / GW; ++k) {
+      for (int k = 0; k < LW / GW; ++k) {
         const int c = w + GW * k;
         if (c >= W) break;
         const int d = __builtin_amdgcn_readlane(dreg, c);
@@ -971,47 +1428,10 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
       if (__ballot(below) != 0ull && lane == 0) S.misc[3] = 1;
     }
     __syncthreads();
-    // The leader wave (wave 0) keeps the row's cumulative histogram in its registers,
-    // scaled from each bin's lattice unit to RFIX per unit of exp(l - m): scale(b) =
-    // 8 exp(arow / LBS - m) 2^(-b log2(e) / LBS). Every wave takes the totals and limits.
-    RowCum rcum;
-    if (w == 0) {
-      const float base = 8.0f * expf(arow * (1.0f / (float)LBS) - m);
-      uint32_t lc = 0u;
-      uint64_t lm = 0ull;
-#pragma unroll
-      for (int q = 0; q < LPL; ++q) {
-        const int bq = LPL * lane + q;
-        rcum.cq(q) = S.rc[bq];
-        const float sc = base * __builtin_amdgcn_exp2f(-(float)bq * (1.44269504f / (float)LBS));
-        rcum.mq(q) = (uint64_t)__double2ull_rn((double)S.rm[bq] * (double)sc);
-        lc += rcum.cq(q);
-        lm += rcum.mq(q);
-      }
-      uint32_t bc = wave_incl_scan_u32(lc) - lc;
-      uint64_t bm = wave_incl_scan_u64(lm) - lm;
-#pragma unroll
-      for (int q = 0; q < LPL; ++q) {
-        bc += rcum.cq(q);
-        bm += rcum.mq(q);
-        rcum.cq(q) = bc;
-        rcum.mq(q) = bm;
-      }
-    }
-    // (LDS values the same in every lane, kept in scalar registers: see uniform_copy)
-    const int rowwin = uniform_copy(S.misc[1] < NBW ? S.misc[1] : NBW);
-    const int rowfull = uniform_copy(S.misc[0] < rowwin ? S.misc[0] : rowwin);
-    const bool anytail = uniform_copy(S.misc[3]) != 0;
-    const int n_all = wave_sum(lane < W ? S.ncnt[lane] : 0);
-    const double S_all = wave_sum(lane < W ? S.sch[lane] : 0.0);
-    const uint64_t S0 = (uint64_t)__double2ull_rn(S_all * RFIX);
-
     const bool topk = p.top_k > 0 && p.top_k < V;
     const bool topp = p.top_p < 1.0f;
     const bool minp = p.min_p > 0.0f;
     const bool icdf = a.noise_mode == STRIM_NOISE_ICDF;
-    // rank-indexed noise needs every kept token's rank
-    if ((p.flags & STRIM_FLAG_NOISE_BY_RANK) && topp && !icdf) return false;
 
     // ---- the leader alone ------------------------------------------------------------
     // A row whose zones are small (the common case) is decided by wave 0 alone, with no
@@ -1020,15 +1440,20 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
     // lanes) and picks within the wave: up to 64 keys by ranks (one key a lane, the zone
     // read as LDS broadcasts), up to SOLO by a radix select in the wave. A zone that needs
     // a chunk's slot region or a collect pass, or holds more than SOLO keys, and Gumbel
-    // draws, go to the cooperative loop below (every wave; it starts over). Both follow
+    // draws, go to gfinal_rest's cooperative loop (every wave; it starts over). Both follow
     // the same decision rules.
     constexpr int SQ = 3, SOLO = SQ * WAVE;  // zone keys a lane holds, a zone's keys
     // (a zone of at most 64 keys starts below 2 SOLO; its rank loop reads up to 7 places
     // past its end)
     static_assert(2 * SOLO + WAVE + 8 <= ZCAP && WAVE + 8 <= GT, "rank loop reads in bounds");
-    bool pfok = true;  // the prefetched candidates are in LDS
     auto solo = [&]() -> int {  // 0 decided, 1 cooperative, 2 exact resolution
       if (!icdf) return 1;
+      // the row's cumulative histogram in the wave's registers, its totals and limits
+      RowCum rcum = row_cum<LW>(S, arow, m);
+      const GTotals tt = row_totals<LW>(S, W);
+      const int rowwin = tt.rowwin, rowfull = tt.rowfull, n_all = tt.n_all;
+      const bool anytail = tt.anytail != 0;
+      const uint64_t S0 = tt.S0;
       int zb0 = -1, zb1 = -1, zn0 = 0, zn1 = 0;
       // lane c's chunk: its top bin's distance below the row's and its window bins
       // written, from its own statistics (the values decide() stores, without the reads)
@@ -1044,7 +1469,7 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
                          cr + rcum.cnt(also) - rcum.cnt(also - 1) <= (uint64_t)SOLO;
         const int bins[2] = {bz, two ? also : -1};
         int off[2], cnt[2], zoo[2], n[2];
-        bool ok = pfok;
+        bool ok = true;
 #pragma unroll
         for (int hh = 0; hh < 2; ++hh) {
           off[hh] = 0;
@@ -1374,263 +1799,24 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
       if (lane == 0) S.misc[5] = verdict;
     }
     __syncthreads();
-    const int verdict = uniform_copy(S.misc[5]);
-    if (verdict == 0) return true;
-    if (verdict == 2) return false;
-
-    // The zone in LDS: up to two bins, zb[h] at [zo[h], zo[h] + zn[h]). A chunk's part of a
-    // bin comes from its prefetched candidates when it lies among them, else from its slot
-    // region; a bin some chunk could not write whole is collected by a streaming pass.
-    int zb[2] = {-1, -1}, zo[2] = {0, 0}, zn[2] = {0, 0}, npick = 0;
-    lds_t<GFinalShared>* Sl = (lds_t<GFinalShared>*)&S;
-    lds_t<GBig>* Gl = (lds_t<GBig>*)&G;
-
-    // The decisions, in order, through one loop (its code is fetched once):
-    //   0 top-k: the k-th key in order (every key counts);
-    //   1 min-p: the kept mass of the keys whose l passes, (double)l - (double)m >= lmp;
-    //   2 top-p: the last kept token is the first whose inclusive mass exceeds P Sk (a
-    //     token is dropped iff the mass before it exceeds P, SpecSampling.swift:62-66);
-    //   3 the icdf draw over the kept keys without the draft.
-    // The leader finds each step's bin and lays out its zone; every wave then loads the
-    // zone and takes part in the pick, and keeps the same state (all of it uniform).
-    // The kept set before top-p: keys <= bound, mass Sk, the bound's bin bbin (NOBIN:
-    // none inside the window); after it: bound1, S1, bb1.
-    uint64_t bound = ~0ull, Sk = S0, bound1 = ~0ull, S1 = S0, wd = 0ull;
-    int bbin = NOBIN, bb1 = NOBIN, xb = NOBIN, token = -1;
-    for (int step = 0; step < 4; ++step) {
-      if (step == 0 && !topk) continue;
-      if (step == 1 && !minp) continue;
-      if (step == 2) {
-        bound1 = bound;
-        S1 = Sk;
-        bb1 = bbin;
-        if (!topp) continue;
-      }
-      if (step == 3) {
-        // the draft of a verify row: kept? its mass and bin
-        if (vdr && l_draft > -INFINITY && ckey(l_draft, draft) <= bound1) {
-          wd = rmass(l_draft, m);
-          xb = row_bin(arow, l_draft);
-        }
-        if (!icdf) break;
-        if (S1 <= wd) {
-          token = arg;  // only the draft kept: the first kept token
-          break;
-        }
-      }
-      // ---- the leader: this step's bin and zone -------------------------------------
-      if (w == 0) {
-        GCmd cmd;
-        cmd.op = GOP_PICK;
-        cmd.load = 0;
-        cmd.also = -1;
-        cmd.by_mass = 1;
-        cmd.excl = -1;
-        cmd.thr = 0.0;
-        cmd.bnd = ~0ull;
-        cmd.bmp = ~0ull;
-        int bz = -1, bfall = NOBIN;
-        uint64_t xw = 0ull;
-        int xbn = NOBIN;
-        if (step == 0) {
-          if (n_all < p.top_k) cmd.op = GOP_SKIP;  // every allowed token is kept
-          cmd.by_mass = 0;
-          cmd.thr = (double)(p.top_k - 1);
-        } else if (step == 1) {
-          const uint32_t flast = minp_last_fkey(m, p.lmp);
-          cmd.bmp = ((uint64_t)flast << 32) | 0xFFFFFFFFull;
-          cmd.op = GOP_SUM;
-          if (cmd.bmp >= bound) {
-            cmd.op = GOP_SKIP;
-          } else {
-            bz = row_bin(arow, fkey_desc_inv(flast));
-            // below the window: with no token below some chunk's window every allowed
-            // token passes (the bound alone is set), else the lattice cannot tell
-            if (bz >= rowwin) cmd.op = anytail ? GOP_FAIL : GOP_BOUND;
-          }
-        } else if (step == 2) {
-          cmd.thr = (double)p.top_p * (double)Sk;
-          cmd.bnd = bound;
-          bfall = bbin;  // the cut lies in the bound's bin when no bin above it crosses
-        } else {
-          cmd.thr = (double)u_draw * (double)(S1 - wd);
-          cmd.bnd = bound1;
-          cmd.excl = draft;
-          xw = wd;
-          xbn = xb;
-          bfall = bb1;
-        }
-        if (cmd.op == GOP_PICK || cmd.op == GOP_SUM) {
-          if (bz < 0) {
-            const int lim = bfall < rowwin ? bfall : rowwin;
-            bz = rcum.find(cmd.by_mass, cmd.thr, lim, xw, xbn);
-            if (bz >= lim) bz = bfall < rowwin ? bfall : NOBIN;
-            // top-p of a sample row: the icdf draw's bin, when it can be told now, is
-            // loaded with the cut's (the kept mass lies between the masses before and
-            // through the cut's bin, so the draw's threshold lies between u times each)
-            if (bz < NOBIN && step == 2 && icdf && !vdr) {
-              const int blo = rcum.find(true, (double)u_draw * (double)rcum.mass(bz - 1), bz + 1, 0ull, NOBIN);
-              const int bhi = rcum.find(true, (double)u_draw * (double)rcum.mass(bz), bz + 1, 0ull, NOBIN);
-              if (blo == bhi && blo <= bz) cmd.also = blo;
-            }
-          }
-          if (bz >= rowwin) {
-            cmd.op = GOP_FAIL;
-          } else if (zb[0] != bz && zb[1] != bz) {
-            if (bz >= rowfull) {
-              cmd.load = 2;
-              cmd.also = -1;
-            } else {
-              const uint64_t cr = rcum.cnt(bz) - rcum.cnt(bz - 1);
-              const int also = cmd.also;
-              const bool two = also >= 0 && also != bz && also < rowfull &&
-                               cr + rcum.cnt(also) - rcum.cnt(also - 1) <= (uint64_t)GT;
-              cmd.also = two ? also : -1;
-              if (cr > (uint64_t)ZCAP) cmd.op = GOP_FAIL;
-              // lane c: chunk c's parts of the bins and their places in the zone
-              const int bins[2] = {bz, cmd.also};
-              int n[2];
-#pragma unroll
-              for (int hh = 0; hh < 2; ++hh) {
-                int cnt = 0, off = 0;
-                if (lane < W && bins[hh] >= 0) {
-                  const int lb = bins[hh] - S.dch[lane];
-                  if (lb >= 0 && lb < S.nbch[lane]) {
-                    off = lb > 0 ? (int)S.pc[lane][lb - 1] : 0;
-                    cnt = (int)S.pc[lane][lb] - off;
-                  }
-                }
-                const int zo_ = (int)wave_incl_scan_u32((uint32_t)cnt) - cnt;
-                n[hh] = __builtin_amdgcn_readlane(zo_ + cnt, WAVE - 1);
-                if (lane < W) {
-                  S.zpo[hh][lane] = off;
-                  S.zpc[hh][lane] = cnt;
-                  S.zpz[hh][lane] = zo_ + (hh ? n[0] : 0);
-                }
-              }
-              cmd.load = 1;
-              cmd.n0 = n[0];
-              cmd.n1 = n[1];
-            }
-          }
-          cmd.c0 = rcum.cnt(bz - 1);
-          cmd.m0 = rcum.mass(bz - 1) - (bz - 1 >= xbn ? xw : 0ull);
-        }
-        cmd.bz = bz;
-        if (lane == 0) S.cmd = cmd;
-      }
-      __syncthreads();
-      const GCmd cmd = uniform_copy(S.cmd);
-      if (cmd.op == GOP_FAIL) return false;
-      if (cmd.op == GOP_SKIP) continue;
-      if (cmd.op == GOP_BOUND) {
-        bound = cmd.bmp;
-        continue;
-      }
-      const int bz = cmd.bz;
-      // ---- every wave: the zone ------------------------------------------------------
-      if (cmd.load == 1) {
-        // wave w copies the parts of chunks w, w + GW, ...: from the prefetched
-        // candidates where they lie among them, else from the chunk's slot region
-        for (int cq = w; cq < W; cq += GW) {
-#pragma unroll
-          for (int hh = 0; hh < 2; ++hh) {
-            const int o = S.zpo[hh][cq], cn = S.zpc[hh][cq], z0 = S.zpz[hh][cq];
-            for (int i = lane; i < cn; i += WAVE) {
-              const int e = o + i;
-              const Cand x = (pfok && e < PF) ? P.pfb[cq * PF + e] : slots[(int64_t)cq * SLOT + e];
-              if (z0 + i < ZCAP) {
-                G.z.zkey[z0 + i] = ckey(x.l, x.id);
-                G.z.zmass[z0 + i] = rmass(x.l, m);
-              }
-            }
-          }
-        }
-        __syncthreads();
-        zb[0] = bz;
-        zo[0] = 0;
-        zn[0] = cmd.n0;
-        zb[1] = cmd.also;
-        zo[1] = cmd.n0;
-        zn[1] = cmd.n1;
-      } else if (cmd.load == 2) {
-        const int n = collect_zone(xa, r, b, j, p, arow - (float)bz, m,
-                                   ZoneLds{(lds_t<uint64_t>*)G.z.zkey, (lds_t<uint64_t>*)G.z.zmass,
-                                           (lds_t<uint32_t>*)P.ccnt, (lds_t<int>*)&S.misc[2]});
-        pfok = false;  // (the pass's history counts took the prefetched candidates' LDS)
-        if (n < 0) return false;
-        zb[0] = bz;
-        zo[0] = 0;
-        zn[0] = n;
-        zb[1] = -1;
-      }
-      const int h = zb[0] == bz ? 0 : 1;
-      if (cmd.op == GOP_SUM) {
-        // min-p: the kept mass is everything before the bound's bin and the zone's keys
-        // up to the bound
-        bound = cmd.bmp;
-        Sk = cmd.m0 + zone_mass_upto(S, G, zo[h], zn[h], bound);
-        bbin = bz;
-        continue;
-      }
-      // ---- the pick: the key whose cumulative interval contains thr ------------------
-      GHit g;
-      {
-        const int np = npick++;
-        if (zn[h] <= RADIX_MIN)
-          g = pick_rank(S, G, np, zo[h], zn[h], cmd.by_mass != 0, cmd.thr, cmd.bnd, cmd.excl,
-                        cmd.c0, cmd.m0);
-        else
-          g = pick_sorted_ool(Sl, Gl, np, zo[h], zn[h], cmd.by_mass != 0, cmd.thr, cmd.bnd,
-                              cmd.excl, cmd.c0, cmd.m0);
-      }
-      if (step == 0) {
-        if (g.key == ~0ull) return false;
-        if (p.flags & STRIM_FLAG_TOPK_KEEP_TIES) {
-          // the keys tied with the k-th one are kept too (same value, same bin)
-          bound = g.key | 0xFFFFFFFFull;
-          Sk = cmd.m0 + zone_mass_upto(S, G, zo[h], zn[h], bound);
-        } else {
-          bound = g.key;
-          Sk = g.mass_before + g.mass;
-        }
-        bbin = bz;
-      } else if (step == 2) {
-        if (g.key != ~0ull) {
-          bound1 = g.key;
-          S1 = g.mass_before + g.mass;
-          bb1 = bz;
-        } else if (bz != bbin) {
-          return false;
-        }
-      } else {
-        if (g.key == ~0ull) return false;
-        token = (int)(uint32_t)g.key;
-      }
-    }
-    if (!icdf) {
-      // Gumbel: every kept candidate (key <= bound1, not the draft)
-      if (bb1 >= rowfull) return false;  // every kept token must be a candidate
-      const bool cand_sorted = (p.flags & STRIM_FLAG_SCORE_NO_LSE) ? topp : (topk || topp);
-      token = gumbel_kept(Sl, slots, a.noise ? a.noise + (int64_t)r * a.noise_stride : nullptr,
-                          W, bb1, bound1, draft, p, m, S1, cand_sorted);
-      if (token < 0) token = arg;  // only the draft kept
-    }
-    const int acc = vdr && ((double)u_acc < (double)wd / (double)S1) ? 1 : 0;
-    finish(STRIM_OK, token, acc, (double)S1 / RFIX, bound1);
-    return true;
+    return uniform_copy(S.misc[5]);
   };
-  if (lat && decide()) return;
-
-  // ---- the exact streaming resolution ----------------------------------------------
-  const XScratch xs = xscratch(G.x.xkey, G.x.xhc, G.x.xcnt, G.x.xu2, S.d, S.u, S.ii);
-  __builtin_amdgcn_s_waitcnt(0);  // (its LDS overlaps the lattice words' and candidates')
-  __syncthreads();
-  const XOut xo =
-      exact_row<GT, false>(xa, r, b, j, p, m, arg, draft, vdr, l_draft, xs, *(lds_t<XState>*)&G.x.x);
+  const int verdict = lat ? decide() : 2;
+  if (verdict == 0) return;
+  GRow g;
+  g.m = m;
+  g.l_draft = l_draft;
+  g.u_draw = u_draw;
+  g.u_acc = u_acc;
+  g.arg = arg;
+  g.draft = draft;
+  g.exact = verdict == 2 ? 1 : 0;
+  const XOut xo = gfinal_rest<LW>(kernel_args(), r, g, (lds_t<GFinalShared<LW>>*)&S,
+                                  (lds_t<GBig<LW>>*)&G, (lds_t<GPf<LW>>*)&P);
   finish(xo.status, xo.token, xo.accept, xo.sig, xo.last_key);
 }
 
+template <int LW>
 hipError_t launch_gfinal(const Args& a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
   const ChunkStat* c = a.s.cstat;
   const unsigned long long* l = a.s.lat;
@@ -1638,9 +1824,11 @@ hipError_t launch_gfinal(const Args& a, hipStream_t st, hipEvent_t e0, hipEvent_
   int wm = a.s.wmax, W = a.W;
   void* args[] = {&c, &l, &sl, &wm, &W, const_cast<Args*>(&a)};
   const dim3 grid((unsigned)a.R), block(GT);
-  const void* k = (const void*)k_gfinal;
+  const void* k = (const void*)k_gfinal<LW>;
   if (e0 || e1) return hipExtLaunchKernel(k, grid, block, args, 0, st, e0, e1, 0);
   return hipLaunchKernel(k, grid, block, args, 0, st);
 }
+// (one object per LW, built in parallel)
+template hipError_t launch_gfinal<STRIM_LW>(const Args&, hipStream_t, hipEvent_t, hipEvent_t);
 
 }  // namespace strim

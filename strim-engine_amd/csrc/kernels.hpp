@@ -39,8 +39,8 @@ constexpr int FCAP_FAST = 4096;  // of which fast rows use at most this many
 constexpr int LBS = 16;          // lattice bins per nat (a power of two: l * LBS is exact)
 constexpr int NBW = 192;         // window bins of a chunk (and of a row, below its top)
 constexpr int LCAP = 256;        // candidates a general row's chunk writes in bin order
-constexpr int LWMAX = 40;        // chunks of a row k_gfinal's lattice path serves
-                                 // (V <= 163,840; wider rows take the exact resolution)
+constexpr int LWNARROW = 40;     // chunks of a row k_gfinal's two builds serve (V <= 163,840,
+constexpr int LWMAX = 64;        // V <= 262,144); wider rows take the exact resolution
 constexpr int LCSH = 51;         // a lattice word: count << LCSH | mass (2^37 per unit of
                                  // exp(l - A / LBS), A the bin's lattice index)
 constexpr uint64_t LMMASK = (1ull << LCSH) - 1ull;

@@ -321,6 +321,34 @@ def test_rank_noise_wide_nucleus(ctx, injected):
     check_sample(ctx, x, p, "bf16", None, None, None, O.NOISE_GUMBEL, noise, label="rank-wide")
 
 
+@pytest.mark.parametrize("V,H", [(5000, 0), (151936, 64), (163841, 0), (248320, 64), (262144, 0)])
+@pytest.mark.parametrize("injected", [False, True])
+def test_rank_noise_candidates(V, H, injected):
+    """Rank-indexed Gumbel noise over nuclei of one token to a few thousand: the kept
+    tokens' ranks from the chunks' candidates, in both builds of k_gfinal (40 and 64
+    chunks); values on a coarse grid (ties, crowded bins), and nuclei past the zone's
+    capacity or the chunks' slots (the exact resolution)."""
+    rng = np.random.default_rng(V + H)
+    B = 6
+    x = rng.normal(0, 2.5, size=(B, V)).astype(np.float32)
+    x[:3] -= 1.1 * np.log(rng.permutation(V) + 1.0).astype(np.float32)
+    x[2] = np.round(x[2] * 4) / 4
+    x[3] = rng.normal(0, 1.0, size=V)      # wide: thousands of kept tokens
+    x[4, rng.integers(V)] = 40.0           # one token holds everything
+    x[5] = np.round(rng.normal(0, 4.0, size=V))
+    p = O.make_params(B, temperature=[0.8, 1.0, 0.7, 1.0, 1.0, 0.5], top_p=[0.95, 0.9, 0.8, 0.3, 0.95, 0.9],
+                      top_k=[0, 0, 0, 0, 0, 1000], presence_penalty=0.5 if H else 0.0,
+                      flags=[7, 2, 7, 3, 7, 6], position=3,
+                      seed=rng.integers(0, 2**63, size=B, dtype=np.uint64))
+    hist = rng.integers(0, V, size=(B, H)).astype(np.int32) if H else None
+    noise = rng.random((B, V + 1), dtype=np.float32) if injected else None
+    with_ctx = ops.Context(0, max_rows=B, max_vocab=V)
+    say(f"rank noise from candidates V={V} H={H} injected={injected}")
+    check_sample(with_ctx, x, p, "bf16", history=hist, noise_mode=O.NOISE_GUMBEL, noise=noise,
+                 label=f"rank noise V={V}")
+    with_ctx.close()
+
+
 @pytest.mark.parametrize("mode", [O.NOISE_ICDF, O.NOISE_GUMBEL])
 def test_minp_slot_overflow(ctx, mode):
     # min-p rows (fast class) over near-flat logits: every chunk overflows its local
