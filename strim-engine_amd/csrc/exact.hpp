@@ -105,6 +105,41 @@ struct XArgs {
   XQ q;
 };
 
+// The streaming passes' view of the launch (collect passes and the exact resolution).
+__device__ __forceinline__ XArgs xargs_of(const Args& a) {
+  XArgs xa;
+  xa.logits = a.logits;
+  xa.row_stride = a.row_stride;
+  xa.dtype = a.dtype;
+  xa.vec_ok = a.vec_ok;
+  xa.V = a.V;
+  xa.H = a.H;
+  xa.verify = a.verify;
+  xa.k = a.k;
+  xa.noise_mode = a.noise_mode;
+  xa.mask = a.mask;
+  xa.mask_stride = a.mask_stride;
+  xa.hist = a.hist;
+  xa.hist_len = a.hist_len;
+  xa.drafts = a.drafts;
+  xa.noise = a.noise;
+  xa.noise_stride = a.noise_stride;
+  xa.has_q = 0;
+  return xa;
+}
+
+// The launch's argument block where the hardware put it, for the functions that are not
+// inlined: its address (two registers) is passed, and they read the fields they use by
+// scalar loads. The block, or the streaming passes' view of it, passed by value goes
+// through scratch memory (4 us a call of the cooperative decisions). Such functions are
+// marked not_tail_called: a call the compiler could make a tail call makes the function
+// save every register it may keep for its caller, some hundred scratch stores and loads
+// a lane (10 us).
+typedef __attribute__((address_space(4))) const Args c_args;
+__device__ __forceinline__ const Args& args_at(uint64_t p) {
+  return *(const Args*)(c_args*)uniform_copy(p);
+}
+
 __device__ __forceinline__ bool x_in(const XUni& u, float l, int id) {
   if (!(l > -INFINITY) || !((double)l - (double)u.m >= u.lmp) || id == u.excl) return false;
   const uint64_t k = ckey(l, id);

@@ -70,44 +70,6 @@ __device__ __forceinline__ int dbin(float m, float l, float scale) {
   return (int)fminf((m - l) * scale, 255.0f);
 }
 
-// Decides a row whose candidates overflow the finalize by the exact streaming
-// resolution (all threads of the workgroup call it). Inlined: only exact_row is an
-// out-of-line call, taking the few launch fields it needs by value, so the 3 KB launch
-// block is never copied to private memory. GQ: see k_finalize.
-template <bool GQ>
-__device__ __forceinline__ void finalize_exact(const Args& a, int r, int b, int j,
-                                            const RowParams& p, float m, int arg, int draft,
-                                            bool vdr, float l_draft, FinalShared& S) {
-  const XScratch xs = xscratch(S.key, S.xhc, S.xcnt, S.xu2, S.d, S.u, S.i);
-  XArgs xa;
-  xa.logits = a.logits;
-  xa.row_stride = a.row_stride;
-  xa.dtype = a.dtype;
-  xa.vec_ok = a.vec_ok;
-  xa.V = a.V;
-  xa.H = a.H;
-  xa.verify = a.verify;
-  xa.k = a.k;
-  xa.noise_mode = a.noise_mode;
-  xa.mask = a.mask;
-  xa.mask_stride = a.mask_stride;
-  xa.hist = a.hist;
-  xa.hist_len = a.hist_len;
-  xa.drafts = a.drafts;
-  xa.noise = a.noise;
-  xa.noise_stride = a.noise_stride;
-  xa.has_q = GQ && vdr ? 1 : 0;
-  __syncthreads();
-  if (GQ && vdr) {
-    xa.q = q_base(a, b * a.k + j);
-    xa.q.mq = S.qmq;
-    xa.q.Z = S.qz;
-  }
-  const XOut xo = exact_row<FTPB, GQ>(xa, r, b, j, p, m, arg, draft, vdr, l_draft, xs,
-                                  *(lds_t<XState>*)&S.x);
-  finish_row(a, r, xo.status, xo.token, xo.accept, xo.sig, m, xo.last_key, PH_DONE);
-}
-
 // One row per 256-thread workgroup, in three phases with two barriers:
 //   1. merge the chunk statistics (max, argmax, flags, k-th value bound G, candidate
 //      counts);
@@ -174,6 +136,36 @@ struct ExactReq {
   int arg, draft;
   float l_draft;
 };
+
+// Decides a row whose candidates overflow the finalize by the exact streaming resolution
+// (all threads of the workgroup call it). Out of line, with the launch's fields and the
+// row's parameters read again: held for it, they took scalar registers from the common
+// path (75 scalar spills to vector lanes, 25 without: B = 1 top-k 14.4 -> 14.1 us a call,
+// the unfiltered one-hot verify 23.0 -> 22.6). GQ: see k_finalize.
+template <bool GQ>
+__attribute__((not_tail_called)) __device__ __noinline__ void finalize_exact(
+    uint64_t kargs, int r, const ExactReq q_in, lds_t<FinalShared>* Sl) {
+  const Args& a = args_at(kargs);
+  const ExactReq q = uniform_copy(q_in);
+  r = __builtin_amdgcn_readfirstlane(r);
+  int b, j;
+  row_bj(a, r, b, j);
+  const bool vdr = a.verify && j < a.k;
+  const RowParams p = load_params(a, b, j);
+  FinalShared& S = *(FinalShared*)Sl;
+  const XScratch xs = xscratch(S.key, S.xhc, S.xcnt, S.xu2, S.d, S.u, S.i);
+  XArgs xa = xargs_of(a);
+  __syncthreads();
+  if (GQ && vdr) {
+    xa.has_q = 1;
+    xa.q = q_base(a, b * a.k + j);
+    xa.q.mq = S.qmq;
+    xa.q.Z = S.qz;
+  }
+  const XOut xo = exact_row<FTPB, GQ>(xa, r, b, j, p, q.m, q.arg, q.draft, vdr, q.l_draft, xs,
+                                      *(lds_t<XState>*)&S.x);
+  finish_row(a, r, xo.status, xo.token, xo.accept, xo.sig, q.m, xo.last_key, PH_DONE);
+}
 
 template <bool GQ>
 __device__ __forceinline__ ExactReq finalize_row(const Args& a, int r, int b, int j,
@@ -771,7 +763,9 @@ __global__ __launch_bounds__(FTPB) void k_finalize(Args a) {
   const ExactReq q = finalize_row<GQ>(a, r, b, j, p, pf, S);
   // one call site for the exact resolution (an out-of-line call), reached by every
   // thread of a row that needs it
-  if (q.need) finalize_exact<GQ>(a, r, b, j, p, q.m, q.arg, q.draft, a.verify && j < a.k, q.l_draft, S);
+  if (q.need)
+    finalize_exact<GQ>((uint64_t)(uintptr_t)__builtin_amdgcn_kernarg_segment_ptr(), r, q,
+                       (lds_t<FinalShared>*)&S);
 }
 
 hipError_t launch_finalize(const Args& a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {

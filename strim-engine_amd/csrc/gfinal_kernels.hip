@@ -432,26 +432,16 @@ __device__ __forceinline__ uint64_t zone_mass_upto(GFinalShared<LW>& S, GBig<LW>
   return tot;
 }
 
-// The launch's argument block where the hardware put it, for the functions that are not
-// inlined: its address (two registers) is passed, and they read the fields they use by
-// scalar loads. The block, or the streaming passes' view of it, passed by value goes
-// through scratch memory (4 us a call of the cooperative decisions). Such functions are
-// marked not_tail_called: a call the compiler could make a tail call makes the function
-// save every register it may keep for its caller, some hundred scratch stores and loads
-// a lane (10 us).
-struct GKernArgs {  // k_gfinal's arguments as the kernel-argument segment lays them out
+// k_gfinal's arguments as the kernel-argument segment lays them out (see args_at).
+struct GKernArgs {
   const ChunkStat* cstat;
   const unsigned long long* lat;
   const Cand* slot;
   int wmax, W;
   Args a;
 };
-typedef __attribute__((address_space(4))) const Args c_args;
 __device__ __forceinline__ uint64_t kernel_args() {
   return (uint64_t)(uintptr_t)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(GKernArgs, a);
-}
-__device__ __forceinline__ const Args& args_at(uint64_t p) {
-  return *(const Args*)(c_args*)uniform_copy(p);
 }
 // Out-of-line forms of the rare paths (their code stays out of the common path's
 // instruction stream; the LDS arrives as an address-space-typed pointer, and only the
@@ -582,29 +572,6 @@ __attribute__((not_tail_called)) __device__ __noinline__ int gumbel_kept(
   }
   block_argmax_score<GT>(bsc, btk, bid, S.d, S.u, S.ii, &S.misc[4]);
   return S.misc[4];
-}
-
-// The streaming passes' view of the launch (collect passes and the exact resolution).
-__device__ __forceinline__ XArgs xargs_of(const Args& a) {
-  XArgs xa;
-  xa.logits = a.logits;
-  xa.row_stride = a.row_stride;
-  xa.dtype = a.dtype;
-  xa.vec_ok = a.vec_ok;
-  xa.V = a.V;
-  xa.H = a.H;
-  xa.verify = a.verify;
-  xa.k = a.k;
-  xa.noise_mode = a.noise_mode;
-  xa.mask = a.mask;
-  xa.mask_stride = a.mask_stride;
-  xa.hist = a.hist;
-  xa.hist_len = a.hist_len;
-  xa.drafts = a.drafts;
-  xa.noise = a.noise;
-  xa.noise_stride = a.noise_stride;
-  xa.has_q = 0;
-  return xa;
 }
 
 // The LDS a collect pass writes (address-space-typed: see lds_t).
