@@ -60,7 +60,7 @@ constexpr size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 // aligned. The general-q verify buffers (dbits .. qarr) are sized only when `verify`.
 struct ScratchLayout {
   size_t cstat, slot, part, rs, cand, nc, dbits, wrank, qpart, qhc, qhm, qst, qpp, qarr, lat,
-      bytes;
+      glist, bytes;
 };
 constexpr ScratchLayout scratch_layout(size_t R, size_t max_vocab, bool verify) {
   const size_t wmax = (max_vocab + CHUNK - 1) / CHUNK;
@@ -84,6 +84,8 @@ constexpr ScratchLayout scratch_layout(size_t R, size_t max_vocab, bool verify) 
   L.qpp = off; off = align_up(off + RQ * QSPLIT * sizeof(QPart), 256);
   L.qarr = off; off = align_up(off + RQ * sizeof(uint32_t), 256);
   L.lat = off; off = align_up(off + R * wmax * NBW * sizeof(unsigned long long), 256);
+  // (rows of one sample group; the no-allocation scratch stays without them)
+  L.glist = off; off = align_up(off + RQ * wmax * CHUNK * sizeof(uint16_t), 256);
   L.bytes = off;
   return L;
 }
@@ -108,6 +110,7 @@ Scratch scratch_at(char* base, const ScratchLayout& L, size_t max_vocab, bool ve
     s.qst = (QStat*)(base + L.qst);
     s.qpp = (QPart*)(base + L.qpp);
     s.qarr = (uint32_t*)(base + L.qarr);
+    s.glist = (uint16_t*)(base + L.glist);
   }
   s.wmax = (int32_t)((max_vocab + CHUNK - 1) / CHUNK);
   return s;

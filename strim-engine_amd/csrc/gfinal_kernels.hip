@@ -98,18 +98,26 @@ struct GCmd {
   int op;           // GOP_*: pick a key, sum the zone's masses up to a bound, skip the
                     // step, only set the bound, or leave the row to the exact resolution
   int load;         // the zone to load first: 0 none (in LDS), 1 from the chunks' parts
-                    // (zpo / zpc / zpz), 2 by a collect pass
+                    // (zpo / zpc / zpz), 2 by a collect pass, 3 from the chunks' window
+                    // lists (the parts of chunks without one: from their slots)
   int bz, also;     // the step's bin; the bin loaded beside it (-1: none)
   int n0, n1;       // the loaded bins' key counts
   int by_mass, excl;
   double thr;
   uint64_t bnd, c0, m0, bmp;
 };
+// The row's totals and limits from the merged lattice.
+struct GTotals {
+  int rowwin, rowfull, anytail, n_all;
+  uint64_t S0;
+};
 template <int LW>
 struct GFinalShared {
   uint16_t pc[LW][NBW];           // per chunk: inclusive count prefix of its window bins
-  uint32_t rc[NBW];               // row bins: counts
-  unsigned long long rm[NBW];     // row bins: masses (RFIX per unit of exp(l - m))
+  // row bins: counts and masses (the lattice's unit); cumulative and scaled to RFIX per unit
+  // of exp(l - m) once the leader has them in registers and passes the row on
+  uint32_t rc[NBW];
+  unsigned long long rm[NBW];
   int nbch[LW];                // per chunk: window bins written
   int ncnt[LW];                // per chunk: allowed tokens
   int dch[LW];                 // per chunk: its top bin's distance below the row's
@@ -125,7 +133,9 @@ struct GFinalShared {
   int32_t tag[2];                 // slots, alternating; tag = the pick's number)
   int zpo[2][LW], zpc[2][LW], zpz[2][LW];  // a zone's parts per chunk: first
                                                     // slot, count, place in the zone
+  uint8_t lst[LW];                // per chunk: 1 its window list is written
   GCmd cmd;                       // the decision loop's current step
+  GTotals tot;                    // for the cooperative decisions, with rc and rm cumulative
   uint32_t prk[GT];               // a pick: each zone key's rank and the mass before it
   unsigned long long pmb[GT];
 };
@@ -276,8 +286,11 @@ __device__ __forceinline__ GHit pick_rank(GFinalShared<LW>& S, GBig<LW>& G, int 
 // <= bound, id != excl), and wave 0 finds the digit d whose interval of cumulative weight
 // (count, or kept mass), from cnt0 / mass0 and the weight below the candidates, holds thr:
 // (double)before(d) <= thr < (double)(before(d) + weight(d)), as pick_rank's rule for one
-// key. The candidates narrow to d until every bit is fixed: about five passes of three
-// barriers for the keys of one lattice bin.
+// key. The candidates narrow to d until at most one wave's worth is left, which wave 0
+// ranks, or every bit is fixed: two passes for the 3,000 keys of a crowded bin. A pass by
+// mass takes no counts, and the lanes of a wave spread over two copies of the histogram: a
+// bin's first digit has few values, so its atomics meet at few addresses (k_gfinal on
+// the wide-nucleus rows, two such picks: 46.6 -> 44.8 us with the three).
 template <int LW>
 __device__ __forceinline__ GHit pick_sorted(GFinalShared<LW>& S, GBig<LW>& G, int np, int z0, int n,
                                             bool by_mass, double thr, uint64_t bound, int excl,
@@ -307,17 +320,16 @@ __device__ __forceinline__ GHit pick_sorted(GFinalShared<LW>& S, GBig<LW>& G, in
   uint64_t bc = cnt0, bm = mass0;  // weights below the candidates
   while (hb >= 0) {
     const int shift = hb >= 7 ? hb - 7 : 0;
-    if (t < 256) {
-      S.prk[t] = 0u;
-      S.pmb[t] = 0ull;
-    }
+    const int copy = (lane & 1) << 8;
+    S.prk[t] = 0u;  // (two copies of 256 digits)
+    S.pmb[t] = 0ull;
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < ZQ; ++q)
       if ((ck[q] & pmask) == prefix) {
         const int d = (int)((ck[q] >> shift) & 255ull);
-        atomicAdd(&S.prk[d], 1u);
-        if (in[q]) atomicAdd(&S.pmb[d], (unsigned long long)km[q]);
+        if (!by_mass) atomicAdd(&S.prk[copy + d], 1u);
+        if (in[q]) atomicAdd(&S.pmb[copy + d], (unsigned long long)km[q]);
       }
     __syncthreads();
     if (w == 0) {
@@ -328,8 +340,8 @@ __device__ __forceinline__ GHit pick_sorted(GFinalShared<LW>& S, GBig<LW>& G, in
       uint64_t lm = 0ull;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        c[i] = S.prk[4 * lane + i];
-        mm[i] = S.pmb[4 * lane + i];
+        c[i] = S.prk[4 * lane + i] + S.prk[256 + 4 * lane + i];
+        mm[i] = S.pmb[4 * lane + i] + S.pmb[256 + 4 * lane + i];
         lc += c[i];
         lm += mm[i];
       }
@@ -372,25 +384,71 @@ __device__ __forceinline__ GHit pick_sorted(GFinalShared<LW>& S, GBig<LW>& G, in
     // every such key shares (a float's low bits that bf16 values leave zero, say) join
     // the prefix without a pass; none left ends the search
     uint64_t vo = 0ull, va = 0ull;  // OR of the keys, OR of their complements
+    int left = 0;                   // the keys under the prefix: this wave's, then all
 #pragma unroll
-    for (int q = 0; q < ZQ; ++q)
-      if ((ck[q] & pmask) == prefix) {
+    for (int q = 0; q < ZQ; ++q) {
+      const bool un = (ck[q] & pmask) == prefix;
+      if (un) {
         vo |= ck[q];
         va |= ~ck[q];
       }
+      left += __popcll(__ballot(un));
+    }
     vo = wave_or_u64(vo);
     va = wave_or_u64(va);
     if (lane == 0) {
       S.u[w] = vo;
       S.u2[GW + w] = va;  // (S.u2[0..1] are read above, before the barrier)
+      S.i[w] = left;
     }
     __syncthreads();  // (also: S.ii and S.u2 are rewritten by the next pass)
     vo = 0ull;
     va = 0ull;
+    int before = 0;  // (the waves before this one)
+    left = 0;
 #pragma unroll
     for (int q = 0; q < GW; ++q) {
       vo |= S.u[q];
       va |= S.u2[GW + q];
+      before += q < w ? S.i[q] : 0;
+      left += S.i[q];
+    }
+    if (left <= WAVE) {
+      // the places of the keys left, gathered for wave 0: one a lane, each compared with
+      // the others through readlane
+#pragma unroll
+      for (int q = 0; q < ZQ; ++q) {
+        const bool un = (ck[q] & pmask) == prefix;
+        const uint64_t bal = __ballot(un);
+        if (un) S.prk[before + lanes_below(bal)] = (uint32_t)(z0 + t + GT * q);
+        before += __popcll(bal);
+      }
+      __syncthreads();
+      if (w == 0) {
+        const int pos = lane < left ? (int)S.prk[lane] : z0;
+        const uint64_t k = G.z.zkey[pos], mk = G.z.zmass[pos];
+        const uint64_t kin = lane < left && k <= bound && (int)(uint32_t)k != excl ? mk : 0ull;
+        uint32_t rk = 0u;
+        uint64_t mb = 0ull;
+        for (int q = 0; q < left; ++q) {
+          const bool lt = rl_u64(k, q) < k;
+          const uint64_t mj = rl_u64(kin, q);
+          rk += lt ? 1u : 0u;
+          mb += lt ? mj : 0ull;
+        }
+        const uint64_t wb = by_mass ? bm + mb : bc + rk;
+        const uint64_t own = by_mass ? kin : 1ull;
+        if (lane < left && own > 0ull && (double)wb <= thr && (double)(wb + own) > thr) {
+          S.res[slot][0] = k;
+          S.res[slot][1] = bc + rk;
+          S.res[slot][2] = bm + mb;
+          S.res[slot][3] = mk;
+          S.tag[slot] = np;
+        }
+      }
+      __syncthreads();
+      if (S.tag[slot] != np) return GHit{~0ull, 0ull, 0ull, 0ull};
+      return GHit{S.res[slot][0], S.res[slot][1], S.res[slot][2], S.res[slot][3]};
     }
     const uint64_t vary = vo & va & ~pmask;
     hb = vary ? 63 - __clzll((long long)vary) : -1;
@@ -467,7 +525,7 @@ __device__ __noinline__ uint32_t minp_last_fkey(float m, double lmp) {
 // candidate entries of bins up to the bound's bin bb, scored in fp64. Returns the token
 // (-1: none kept but the draft). by_rank: a token's noise is that of its rank in the
 // row's order. The entries are first laid out by row bin (each bin's first place from the
-// row's counts, S.rc, a token's place in its bin by an atomic), and a token's rank is its
+// row's cumulative counts, a token's place in its bin by an atomic), and a token's rank is its
 // bin's first place plus the smaller keys of its bin, so a nucleus of a few thousand
 // tokens needs no sort; past ZCAP entries: -2, the exact resolution.
 template <int LW>
@@ -499,20 +557,6 @@ __attribute__((not_tail_called)) __device__ __noinline__ int gumbel_kept(
     const int zof = (int)wave_incl_scan_u32((uint32_t)lim) - lim;
     if (lane < W) S.zoff[lane] = zof;
     if (lane == W - 1) S.zoff[W] = zof + lim;
-    if (by_rank) {  // the row bins' counts become their exclusive prefixes
-      uint32_t c[LPL], tot = 0u;
-#pragma unroll
-      for (int q = 0; q < LPL; ++q) {
-        c[q] = S.rc[LPL * lane + q];
-        tot += c[q];
-      }
-      uint32_t run = wave_incl_scan_u32(tot) - tot;
-#pragma unroll
-      for (int q = 0; q < LPL; ++q) {
-        S.rc[LPL * lane + q] = run;
-        run += c[q];
-      }
-    }
   }
   if (by_rank && t < NBW) S.prk[t] = 0u;
   __syncthreads();
@@ -537,7 +581,7 @@ __attribute__((not_tail_called)) __device__ __noinline__ int gumbel_kept(
     const uint64_t k = ckey(x.l, x.id);
     if (by_rank) {  // (every entry: those of the bound's bin past it rank after it)
       const int bq = row_bin(arow, x.l);
-      G.z.zkey[S.rc[bq] + atomicAdd(&S.prk[bq], 1u)] = k;
+      G.z.zkey[(bq > 0 ? S.rc[bq - 1] : 0u) + atomicAdd(&S.prk[bq], 1u)] = k;
       continue;
     }
     if (k > bound || x.id == draft) continue;
@@ -558,7 +602,7 @@ __attribute__((not_tail_called)) __device__ __noinline__ int gumbel_kept(
       if (k > bound) continue;
       const float l = key_l(k);
       const int bq = row_bin(arow, l);
-      const int z0 = (int)S.rc[bq], z1 = z0 + (int)S.prk[bq];
+      const int z0 = bq > 0 ? (int)S.rc[bq - 1] : 0, z1 = z0 + (int)S.prk[bq];
       int rank = z0;
       for (int q = z0; q < z1; ++q) rank += G.z.zkey[q] < k ? 1 : 0;
       const float u = noise ? noise[rank] : philox_uniform(pkey, (uint64_t)rank);
@@ -806,12 +850,7 @@ __attribute__((not_tail_called)) __device__ __noinline__ int collect_zone(uint64
   return n <= ZCAP ? n : -1;
 }
 
-// The row's totals and limits from the merged lattice (every lane; scalar: see
-// uniform_copy).
-struct GTotals {
-  int rowwin, rowfull, anytail, n_all;
-  uint64_t S0;
-};
+// (every lane; scalar: see uniform_copy)
 template <int LW>
 __device__ __forceinline__ GTotals row_totals(GFinalShared<LW>& S, int W) {
   const int lane = threadIdx.x & (WAVE - 1);
@@ -886,9 +925,15 @@ __attribute__((not_tail_called)) __device__ __noinline__ XOut gfinal_rest(uint64
   const float arow = floorf(m * (float)LBS);
   XOut out{STRIM_OK, -1, 0, 0.0, 0ull};
   auto decide = [&]() -> bool {
-    const GTotals tt = row_totals<LW>(S, W);
+    const GTotals tt = uniform_copy(S.tot);
     RowCum rcum;
-    if (w == 0) rcum = row_cum<LW>(S, arow, m);
+    if (w == 0) {
+#pragma unroll
+      for (int q = 0; q < LPL; ++q) {
+        rcum.cq(q) = S.rc[LPL * lane + q];
+        rcum.mq(q) = S.rm[LPL * lane + q];
+      }
+    }
     const int rowwin = tt.rowwin, rowfull = tt.rowfull, n_all = tt.n_all;
     const bool anytail = tt.anytail != 0;
     const uint64_t S0 = tt.S0;
@@ -897,6 +942,21 @@ __attribute__((not_tail_called)) __device__ __noinline__ XOut gfinal_rest(uint64
     const bool minp = p.min_p > 0.0f;
     const bool icdf = a.noise_mode == STRIM_NOISE_ICDF;
     bool pfok = true;  // the prefetched candidates are in LDS
+    // (leader) the row bins whose tokens the slots or the window lists hold, read once a
+    // bin past the slots is asked for
+    int listfull = -1;
+    auto lists = [&]() {
+      if (listfull >= 0) return;
+      int lim = NBW, has = 0;
+      if (lane < W) {
+        const ChunkStat& cs = a.s.cstat[(int64_t)r * a.s.wmax + lane];
+        has = a.s.glist != nullptr && r < MAXP && cs.n > 0 && cs.g2 != 0.0f ? 1 : 0;
+        if (cs.n > 0 && !has && cs.ncand < cs.ncand2) lim = min(NBW, S.dch[lane] + (int)cs.ncand);
+        S.lst[lane] = (uint8_t)has;
+      }
+      lim = wave_min_i(lim);
+      listfull = uniform_copy(min(lim, rowwin));
+    };
     // The zone in LDS: up to two bins, zb[h] at [zo[h], zo[h] + zn[h]). A chunk's part of a
     // bin comes from its prefetched candidates when it lies among them, else from its slot
     // region; a bin some chunk could not write whole is collected by a streaming pass.
@@ -994,13 +1054,18 @@ __attribute__((not_tail_called)) __device__ __noinline__ XOut gfinal_rest(uint64
           if (bz >= rowwin) {
             cmd.op = GOP_FAIL;
           } else if (zb[0] != bz && zb[1] != bz) {
+            int full = rowfull;
             if (bz >= rowfull) {
+              lists();
+              full = listfull;
+            }
+            if (bz >= full) {
               cmd.load = 2;
               cmd.also = -1;
             } else {
               const uint64_t cr = rcum.cnt(bz) - rcum.cnt(bz - 1);
               const int also = cmd.also;
-              const bool two = also >= 0 && also != bz && also < rowfull &&
+              const bool two = also >= 0 && also != bz && also < full &&
                                cr + rcum.cnt(also) - rcum.cnt(also - 1) <= (uint64_t)GT;
               cmd.also = two ? also : -1;
               if (cr > (uint64_t)ZCAP) cmd.op = GOP_FAIL;
@@ -1025,7 +1090,7 @@ __attribute__((not_tail_called)) __device__ __noinline__ XOut gfinal_rest(uint64
                   S.zpz[hh][lane] = zo_ + (hh ? n[0] : 0);
                 }
               }
-              cmd.load = 1;
+              cmd.load = bz < rowfull && (!two || also < rowfull) ? 1 : 3;
               cmd.n0 = n[0];
               cmd.n1 = n[1];
             }
@@ -1066,6 +1131,73 @@ __attribute__((not_tail_called)) __device__ __noinline__ XOut gfinal_rest(uint64
               if (z0 + i < ZCAP) {
                 G.z.zkey[z0 + i] = ckey(x.l, x.id);
                 G.z.zmass[z0 + i] = rmass(x.l, m);
+              }
+            }
+          }
+        }
+        __syncthreads();
+        zb[0] = bz;
+        zo[0] = 0;
+        zn[0] = cmd.n0;
+        zb[1] = cmd.also;
+        zo[1] = cmd.n0;
+        zn[1] = cmd.n1;
+      } else if (cmd.load == 3) {
+        // (instead of a collect pass: k_gfinal on the wide-nucleus rows 84 -> 46.6 us.)
+        // Wave w gathers the parts of chunks w, w + GW, ...: a token's place in its chunk
+        // from the window list, then its logit (the round trips of all its chunks' first
+        // 2 WAVE tokens overlap), l = x / T as k_stream formed it
+        constexpr int KC = LW / GW;
+        auto put = [&](int z, float l, int id) {
+          if (z < ZCAP) {
+            G.z.zkey[z] = ckey(l, id);
+            G.z.zmass[z] = rmass(l, m);
+          }
+        };
+        const glb_t<const uint16_t>* gl =
+            (const glb_t<const uint16_t>*)(a.s.glist + (int64_t)r * a.s.wmax * CHUNK);
+        const int64_t xb = (int64_t)r * a.row_stride;
+        auto logit = [&](int id) -> float {
+          return a.dtype == STRIM_DTYPE_BF16
+                     ? bf16_to_f32(((const glb_t<const uint16_t>*)a.logits)[xb + id])
+                     : ((const glb_t<const float>*)a.logits)[xb + id];
+        };
+#pragma unroll
+        for (int hh = 0; hh < 2; ++hh) {
+          if (hh == 1 && cmd.also < 0) continue;
+          int id[KC][2];
+          float x[KC][2];
+#pragma unroll
+          for (int k = 0; k < KC; ++k) {
+            const int cq = min(w + GW * k, W - 1), o = S.zpo[hh][cq];
+            const int cn = w + GW * k < W && S.lst[cq] ? S.zpc[hh][cq] : 0;
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+              const int i = lane + WAVE * q;
+              id[k][q] = i < cn ? cq * CHUNK + (int)gl[(int64_t)cq * CHUNK + o + i] : -1;
+            }
+          }
+#pragma unroll
+          for (int k = 0; k < KC; ++k)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) x[k][q] = logit(max(id[k][q], 0));
+#pragma unroll
+          for (int k = 0; k < KC; ++k)
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+              if (id[k][q] >= 0)
+                put(S.zpz[hh][w + GW * k] + lane + WAVE * q, x[k][q] / p.T, id[k][q]);
+          for (int cq = w; cq < W; cq += GW) {
+            const int o = S.zpo[hh][cq], cn = S.zpc[hh][cq], z0 = S.zpz[hh][cq];
+            if (S.lst[cq]) {
+              for (int i = 2 * WAVE + lane; i < cn; i += WAVE) {
+                const int ix = cq * CHUNK + (int)gl[(int64_t)cq * CHUNK + o + i];
+                put(z0 + i, logit(ix) / p.T, ix);
+              }
+            } else {
+              for (int i = lane; i < cn; i += WAVE) {
+                const glb_t<const Cand>& y = ((const glb_t<const Cand>*)slots)[(int64_t)cq * SLOT + o + i];
+                put(z0 + i, y.l, y.id);
               }
             }
           }
@@ -1402,22 +1534,20 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
 
     // ---- the leader alone ------------------------------------------------------------
     // A row whose zones are small (the common case) is decided by wave 0 alone, with no
-    // workgroup barrier: it lays out each zone from the prefetched candidates (each
-    // place's source recorded by its chunk's lane, then the keys and masses built by all
-    // lanes) and picks within the wave: up to 64 keys by ranks (one key a lane, the zone
-    // read as LDS broadcasts), up to SOLO by a radix select in the wave. A zone that needs
-    // a chunk's slot region or a collect pass, or holds more than SOLO keys, and Gumbel
-    // draws, go to gfinal_rest's cooperative loop (every wave; it starts over). Both follow
-    // the same decision rules.
+    // workgroup barrier: it lays out each zone from the prefetched candidates or the
+    // chunks' slot regions (each place's source recorded by its chunk's lane, then the keys
+    // and masses built by all lanes) and picks within the wave: up to 64 keys by ranks (one
+    // key a lane, the zone read as LDS broadcasts), up to SOLO by a radix select in the
+    // wave. A zone past the slots, or of more than SOLO keys, and Gumbel draws, go to
+    // gfinal_rest's cooperative loop (every wave; it starts over). Both follow the same
+    // decision rules.
     constexpr int SQ = 3, SOLO = SQ * WAVE;  // zone keys a lane holds, a zone's keys
     // (a zone of at most 64 keys starts below 2 SOLO; its rank loop reads up to 7 places
     // past its end)
     static_assert(2 * SOLO + WAVE + 8 <= ZCAP && WAVE + 8 <= GT, "rank loop reads in bounds");
-    auto solo = [&]() -> int {  // 0 decided, 1 cooperative, 2 exact resolution
+    auto solo = [&](const RowCum& rcum, const GTotals& tt) -> int {  // 0 decided, 1
+      // cooperative, 2 exact resolution
       if (!icdf) return 1;
-      // the row's cumulative histogram in the wave's registers, its totals and limits
-      RowCum rcum = row_cum<LW>(S, arow, m);
-      const GTotals tt = row_totals<LW>(S, W);
       const int rowwin = tt.rowwin, rowfull = tt.rowfull, n_all = tt.n_all;
       const bool anytail = tt.anytail != 0;
       const uint64_t S0 = tt.S0;
@@ -1436,7 +1566,7 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
                          cr + rcum.cnt(also) - rcum.cnt(also - 1) <= (uint64_t)SOLO;
         const int bins[2] = {bz, two ? also : -1};
         int off[2], cnt[2], zoo[2], n[2];
-        bool ok = true;
+        bool far = false;  // a part lies past the chunk's prefetched candidates
 #pragma unroll
         for (int hh = 0; hh < 2; ++hh) {
           off[hh] = 0;
@@ -1450,17 +1580,19 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
           }
           zoo[hh] = (int)wave_incl_scan_u32((uint32_t)cnt[hh]) - cnt[hh];
           n[hh] = __builtin_amdgcn_readlane(zoo[hh] + cnt[hh], WAVE - 1);
-          ok = ok && off[hh] + cnt[hh] <= PF;
+          far = far || off[hh] + cnt[hh] > PF;
         }
-        if (__ballot(!ok) != 0ull || n[0] + n[1] > SOLO) return 1;
+        if (n[0] + n[1] > SOLO) return 1;
+        far = __ballot(far) != 0ull;
         zoo[1] += n[0];
-        // each zone place's source in the prefetched candidates, c PF + its place in
-        // chunk c's part: lane c writes its part's (a few stores each), then every lane
+        // each zone place's source, chunk c and its place among c's candidates: lane c
+        // writes its part's (a few stores each), then every lane
         // builds the keys and masses of places lane, lane + 64, ... (S.prk is idle here)
         lds_t<uint32_t>* src = (lds_t<uint32_t>*)S.prk;
+        const int str = far ? SLOT : PF;  // (the chunks' stride where they are read)
 #pragma unroll
         for (int hh = 0; hh < 2; ++hh)
-          for (int i = 0; i < cnt[hh]; ++i) src[zoo[hh] + i] = (uint32_t)(lane * PF + off[hh] + i);
+          for (int i = 0; i < cnt[hh]; ++i) src[zoo[hh] + i] = (uint32_t)(lane * str + off[hh] + i);
         __builtin_amdgcn_wave_barrier();
         // (at most SOLO places: every lane's SQ sources read first, then their candidates)
         const int ntot = n[0] + n[1];
@@ -1471,8 +1603,15 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
           si[q] = src[i < ntot ? i : 0];
         }
         Cand xc[SQ];
+        if (!far) {
 #pragma unroll
-        for (int q = 0; q < SQ; ++q) xc[q] = P.pfb[lane + WAVE * q < ntot ? si[q] : 0u];
+          for (int q = 0; q < SQ; ++q) xc[q] = P.pfb[lane + WAVE * q < ntot ? si[q] : 0u];
+        } else {
+          // from the slot regions, one more round trip (a row left to the cooperative
+          // decisions for such a part took 3 us more)
+#pragma unroll
+          for (int q = 0; q < SQ; ++q) xc[q] = slots[lane + WAVE * q < ntot ? si[q] : 0u];
+        }
 #pragma unroll
         for (int q = 0; q < SQ; ++q) {
           const int i = lane + WAVE * q;
@@ -1762,7 +1901,18 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
       return 0;
     };
     if (w == 0) {
-      const int verdict = solo();
+      // the row's cumulative histogram in the wave's registers, its totals and limits
+      RowCum rcum = row_cum<LW>(S, arow, m);
+      const GTotals tt = row_totals<LW>(S, W);
+      const int verdict = solo(rcum, tt);
+      if (verdict == 1) {
+#pragma unroll
+        for (int q = 0; q < LPL; ++q) {
+          S.rc[LPL * lane + q] = rcum.cq(q);
+          S.rm[LPL * lane + q] = rcum.mq(q);
+        }
+        if (lane == 0) S.tot = tt;
+      }
       if (lane == 0) S.misc[5] = verdict;
     }
     __syncthreads();

@@ -68,7 +68,7 @@ struct ChunkStat {
   int32_t arg;     // first id reaching m
   uint32_t ncand;  // fast rows: candidates in the chunk's slot region (> SLOT: overflow);
                    // general rows: window bins whose tokens are all written (nfull)
-  float g2;        // (unused)
+  float g2;        // general rows: nonzero when the chunk's window list is written (glist)
   uint32_t ncand2; // general rows: window bins with lattice words written (nb: the last
                    // non-empty bin + 1); LNONE when the lattice cannot hold the row
   uint32_t pad_;
@@ -144,6 +144,9 @@ struct Scratch {
   unsigned long long* lat;        // [rows][wmax][NBW] general rows: per window bin of the
                                   // chunk, its inclusive count prefix << LCSH | its mass
                                   // (2^37 per unit of exp(l - A / LBS), A the bin's index)
+  uint16_t* glist;                // [min(rows, MAXP)][wmax][CHUNK] general rows whose nucleus
+                                  // outgrows the slots: every window token's place in the
+                                  // chunk, in bin order (null: none are written)
   int32_t wmax;
 };
 

@@ -321,6 +321,36 @@ def test_rank_noise_wide_nucleus(ctx, injected):
     check_sample(ctx, x, p, "bf16", None, None, None, O.NOISE_GUMBEL, noise, label="rank-wide")
 
 
+@pytest.mark.parametrize("V,B", [(4097, 6), (40001, 6), (151936, 6), (151936, 36), (151936, 70),
+                                 (248320, 6)])
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+def test_wide_nuclei_window_lists(V, B, dtype):
+    """Nuclei past the chunks' slots, whose cut or draw bin is gathered from the window
+    lists: top-p, large top-k and no filter, masks, tied values, aligned and odd rows, one
+    chunk and many, rows without a list in the same batch (peaked, penalised, past the 64
+    rows of a group), and bins past a zone's capacity (the exact resolution)."""
+    rng = np.random.default_rng(V + B)
+    x = rng.normal(0, 1.0, size=(B, V)).astype(np.float32)
+    x[1] *= 2.0
+    x[2] = np.round(x[2] * 8) / 8
+    x[3, rng.integers(V)] = 30.0  # peaked
+    x[4] *= 0.3                   # near-uniform: bins of thousands of tokens
+    p = O.make_params(B, temperature=np.resize([1.0, 0.8, 1.0, 1.0, 0.7, 1.1], B),
+                      top_p=np.resize([0.95, 0.9, 0.8, 0.95, 0.9, 1.0], B),
+                      top_k=np.resize([0, 0, 0, 0, 0, 0, V // 2, 300], B),
+                      seed=rng.integers(0, 2**63, size=B, dtype=np.uint64), position=9)
+    mask = W.pack_mask(rng.random((B, V)) < 0.7)
+    hist = rng.integers(0, V, size=(B, 16)).astype(np.int32)
+    noise = rng.random((B, 2), dtype=np.float32)
+    c = ops.Context(0, max_rows=B, max_vocab=V)
+    say(f"wide nuclei V={V} B={B} {dtype}")
+    check_sample(c, x, p, dtype, noise=noise, probs=B <= 6, label=f"wide V={V} B={B}")
+    check_sample(c, x, p, dtype, mask=mask, noise=noise, probs=False, label=f"wide masked V={V} B={B}")
+    p["presence_penalty"] = np.resize([0.0, 0.5], B)
+    check_sample(c, x, p, dtype, history=hist, noise=noise, probs=False, label=f"wide pen V={V} B={B}")
+    c.close()
+
+
 @pytest.mark.parametrize("V,H", [(5000, 0), (151936, 64), (163841, 0), (248320, 64), (262144, 0)])
 @pytest.mark.parametrize("injected", [False, True])
 def test_rank_noise_candidates(V, H, injected):
