@@ -92,9 +92,13 @@ struct RowPre {
   Cand c[PRE_E];
   float n0, n1, l_draft;
   int draft;
+  QPart qp;                // general-q draft rows: lane q's slice of the draft row
+  int qbad;                // (lane q: the table check of slice q)
+  uint32_t qdw, qdr;       // the draft's table word and its rank
   int kd;          // speculative depth K per chunk region (even)
   uint32_t kmag;   // entry e lies in region umulhi(e, kmag) = e / K
 };
+template <bool GQ>
 __device__ __forceinline__ RowPre prefetch_row(const Args& a, int r, int b, int j) {
   RowPre f;
   const int t = threadIdx.x;
@@ -126,6 +130,18 @@ __device__ __forceinline__ RowPre prefetch_row(const Args& a, int r, int b, int 
   f.draft = vdr ? d : -1;
   const float ld = rsp->l_draft;
   f.l_draft = vdr ? ld : -INFINITY;
+  if constexpr (GQ) {
+    // the draft distribution's slices, one a lane, and the draft's membership: requested
+    // with the rest, so the merge and q(draft) wait for no round trip of their own (read
+    // when used, they cost a filtered round 26.5 us against 24.6)
+    const int lane = t & (WAVE - 1), q = lane < QSPLIT ? lane : 0;
+    const int qr = vdr ? b * a.k + j : 0;
+    f.qp = a.s.qpp[(size_t)qr * QSPLIT + q];
+    f.qbad = a.s.qpp[q].bad;
+    const int dq = (unsigned)f.draft < (unsigned)a.V ? f.draft : 0;
+    f.qdw = a.s.dbits[dq >> 5];
+    f.qdr = a.s.wrank[dq >> 5];
+  }
   return f;
 }
 
@@ -251,33 +267,25 @@ __device__ __forceinline__ ExactReq finalize_row(const Args& a, int r, int b, in
     finish_row(a, r, STRIM_OK, arg, vdr && arg == draft, 1.0, m, 0ull, PH_DONE);
     return done;
   }
-  XQ xq;  // (general-q draft rows: their q, valid in wave 0)
+  XQ xq;  // (general-q draft rows: their q)
+  float qd_v = 0.0f;  // (their draft's v = draft logit / T)
   const bool gq = GQ && vdr;
   if (gq) {
     // general-q draft row: the draft distribution from k_qprep's slices (its maximum, the
     // draft's table index, fp64 Z = sum exp(v - mq)), published for the residual draw;
     // the draft must be in a valid table (the first draft row's slices checked it)
     const int qr = b * a.k + j;
-    const QPart* pp = a.s.qpp + (size_t)qr * QSPLIT;
-    float mq = -INFINITY;
-    int td = -1, bad = 0;
-#pragma unroll
-    for (int q = 0; q < QSPLIT; ++q) {
-      mq = fmaxf(mq, pp[q].m);
-      td = max(td, pp[q].td);
-      bad |= a.s.qpp[q].bad;
-    }
-    // Z = sum over the slices of z exp(m - mq): one slice per lane of wave 0
-    double z = 0.0;
-    if (w == 0) {
-      const QPart& pq = pp[lane < QSPLIT ? lane : 0];
-      z = wave_sum(lane < QSPLIT && pq.m > -INFINITY ? pq.z * exp((double)pq.m - (double)mq)
-                                                     : 0.0);
-      if (t == 0) {
-        a.s.qst[qr] = QStat{mq, td, z};
-        S.qz = z;
-        S.qmq = mq;
-      }
+    // (every wave merges the slices its lanes hold; Z is wave 0's to use)
+    const bool sl = lane < QSPLIT;
+    const float mq = wave_max_f(sl ? pf.qp.m : -INFINITY);
+    const int td = wave_max_i(sl ? pf.qp.td : -1);
+    const int bad = wave_or_i(sl ? pf.qbad : 0);
+    const double z = wave_sum(sl && pf.qp.m > -INFINITY
+                                  ? pf.qp.z * exp((double)pf.qp.m - (double)mq) : 0.0);
+    if (t == 0) {
+      a.s.qst[qr] = QStat{mq, td, z};
+      S.qz = z;
+      S.qmq = mq;
     }
     if (bad || td < 0) {
       finish_row(a, r, STRIM_EINVAL, -1, 0, 0.0, m, 0ull, PH_DONE);
@@ -286,6 +294,8 @@ __device__ __forceinline__ ExactReq finalize_row(const Args& a, int r, int b, in
     xq = q_base(a, qr);
     xq.mq = mq;
     xq.Z = z;
+    // q(draft): its logit is requested here, used after the candidates are decided
+    if (p.cls == CLS_FAST) qd_v = xq_v(xq, draft, pf.qdw, pf.qdr);
     // fast rows go on to the candidates below. Unfiltered rows: the grid-wide residual draw
     // (qres_kernels.hip); the others: k_final's exact resolution (the row's first maximum
     // is kept as the fallback token)
@@ -313,12 +323,9 @@ __device__ __forceinline__ ExactReq finalize_row(const Args& a, int r, int b, in
         const double sig = (double)Sq / XFIX;
         const double w_d = l_draft > -INFINITY ? exp((double)l_draft - (double)m) : 0.0;
         double ratio = w_d / sig;
-        const uint32_t dw = a.s.dbits[draft >> 5];
-        const bool in_tab = (dw >> (draft & 31)) & 1u;
+        const bool in_tab = (pf.qdw >> (draft & 31)) & 1u;
         const double qd =
-            in_tab ? exp((double)xq_v(q_base(a, qr), draft, dw, a.s.wrank[draft >> 5]) -
-                         (double)mq) / z
-                   : 0.0;
+            in_tab ? exp((double)xq_v(xq, draft, pf.qdw, pf.qdr) - (double)mq) / z : 0.0;
         ratio = qd > 0.0 ? ratio / qd : (ratio > 0.0 ? INFINITY : 0.0);
         const float ua =
             a.noise ? pf.n1
@@ -628,7 +635,7 @@ __device__ __forceinline__ ExactReq finalize_row(const Args& a, int r, int b, in
     // and the draft logit each, one candidate a lane at the usual top-k) and the row ends
     // here. It went to k_final's streaming resolution, six passes of one workgroup over the
     // row: V = 151,936, B = 4, k = 3, Vd = 32,768, top-k 20, top-p 0.95 took 587 us a
-    // round, and takes 26.9 us with the lookups.
+    // round, and takes 24.6 us with the lookups.
     auto qprob = [&](int q) { return q < k1 ? xq_prob(xq, (int)(uint32_t)keys[q]) : 0.0; };
     const double q0 = qprob(p0);
     if (a.noise_mode == STRIM_NOISE_ICDF) {
@@ -683,7 +690,8 @@ __device__ __forceinline__ ExactReq finalize_row(const Args& a, int r, int b, in
       if (token < 0) token = (int)(uint32_t)keys[0];  // p <= q everywhere
     }
     // accept iff u < p(d) / q(d)
-    const double qd = xq_prob(xq, draft);
+    const double qd =
+        (pf.qdw >> (draft & 31)) & 1u ? exp((double)qd_v - (double)xq.mq) / xq.Z : 0.0;
     const double pd = w_d / S_kept;
     const double ratio = qd > 0.0 ? pd / qd : (pd > 0.0 ? INFINITY : 0.0);
     finish_row(a, r, STRIM_OK, token, (double)u_acc < ratio ? 1 : 0, S_kept, m, last_key, PH_DONE);
@@ -756,7 +764,7 @@ __global__ __launch_bounds__(FTPB) void k_finalize(Args a) {
   const int r = blockIdx.x;
   int b, j;
   row_bj(a, r, b, j);
-  const RowPre pf = prefetch_row(a, r, b, j);
+  const RowPre pf = prefetch_row<GQ>(a, r, b, j);
   const RowParams p = load_params(a, b, j);
   // the general rows are k_gfinal's
   if (gfinal_row(a.p[b], a.V, a.noise_mode, GQ && j < a.k)) return;
