@@ -29,7 +29,7 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
-constexpr int HN_T = 256;               // k_head_norm threads
+constexpr int HN_T = 1024;              // k_head_norm threads
 constexpr int HG_W = 4;                 // k_head_gemv waves per workgroup
 constexpr int HG_MT = 2;                // 16-row vocabulary tiles per wave
 constexpr int HG_KS = 128;              // K elements per step (four MFMAs of K 32)
@@ -48,8 +48,14 @@ __global__ __launch_bounds__(HN_T) void k_head_norm(const uint16_t* x, int64_t x
   const int b = blockIdx.x, t = threadIdx.x;
   const uint16_t* xr = x + (int64_t)b * x_stride;
   double ss = 0.0;
+  // A row's time is its chain of round trips: the first 8 HN_T elements' row and weight
+  // pieces (all of them up to K = 8,192) are requested together and held, so the
+  // normalisation after the sum waits for no second trip (K = 5,120: 6.0 -> 4.6 us; 256
+  // threads read the row twice).
+  const int k0 = 8 * t < K ? 8 * t : 0;
+  const uint4 q0 = *(const uint4*)(xr + k0), g0 = *(const uint4*)(w + k0);
   for (int k = 8 * t; k < K; k += 8 * HN_T) {
-    const uint4 q = *(const uint4*)(xr + k);
+    const uint4 q = k == k0 ? q0 : *(const uint4*)(xr + k);
     const uint32_t wd[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -65,8 +71,8 @@ __global__ __launch_bounds__(HN_T) void k_head_norm(const uint16_t* x, int64_t x
   for (int q = 0; q < HN_T / WAVE; ++q) tot += s_d[q];
   const float inv = 1.0f / sqrtf((float)(tot / (double)K) + eps);
   for (int k = 8 * t; k < K; k += 8 * HN_T) {
-    const uint4 q = *(const uint4*)(xr + k);
-    const uint4 g = *(const uint4*)(w + k);
+    const uint4 q = k == k0 ? q0 : *(const uint4*)(xr + k);
+    const uint4 g = k == k0 ? g0 : *(const uint4*)(w + k);
     const uint32_t xd[4] = {q.x, q.y, q.z, q.w}, gd[4] = {g.x, g.y, g.z, g.w};
     uint32_t o[4];
 #pragma unroll
