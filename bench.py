@@ -427,12 +427,12 @@ def head_bench(torch, ops, dev, ctx, args, w1, m1, hl, B=8, K=5120):
     torch.cuda.empty_cache()
     return {
         "workload": f"final RMSNorm + dense bf16 lm_head: hidden [{B},{K}] x lm_head [{V},{K}] "
-                    "-> bf16 logits (k_head_norm + k_head_gemv, MFMA 16x16x32 bf16)",
+                    "-> bf16 logits (k_head_norm + k_head_split, MFMA 16x16x32 bf16)",
         "us_per_call": round(ush, 2), "steps": kh,
         "roofline": {"bound": "hbm", "achieved": round(byt / (ush * 1e-6) / 1e9, 1),
                      "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(byt / (ush * 1e-6) / 1e9 / HBM_PEAK_GBS, 4),
-                     "bytes_per_call": int(byt), "kernel": "k_head_norm + k_head_gemv"},
+                     "bytes_per_call": int(byt), "kernel": "k_head_norm + k_head_split"},
         "mfma_tflops": round(flops / (ush * 1e-6) / 1e12, 2),
         "then_n1_chain_us_per_step": round(usc, 2),
         "sampler_share_us": round(usc - ush, 2),

@@ -702,10 +702,10 @@ int strim_head_greedy(strim_ctx* ctx, void* stream, const void* hidden, int64_t 
                     V, out_logits, out_stride))
     return STRIM_EINVAL;
   if (B > ctx->max_rows || V > ctx->max_vocab) return STRIM_ECAPACITY;
-  // the tile maxima [B][ceil(V / 128)] go to the context's candidate slots (stream-ordered
-  // with every other call on the context; they need B * V / 16 bytes, the slots hold
+  // the tile maxima [B][up to ceil(V / 32)] go to the context's candidate slots (stream-ordered
+  // with every other call on the context; they need at most B * V / 4 bytes, the slots hold
   // max_rows * max_vocab bytes)
-  static_assert(sizeof(Cand) * SLOT >= (CHUNK / 128) * sizeof(uint2), "tile maxima fit the slots");
+  static_assert(sizeof(Cand) * SLOT >= (CHUNK / 32) * sizeof(uint2), "tile maxima fit the slots");
   uint2* tbest = (uint2*)ctx->s.slot;
   const bool vo = out_logits && ((uintptr_t)out_logits & 7u) == 0 && out_stride % 4 == 0;
   const hipError_t e = launch_head(hidden, hidden_stride, B, K, norm_weight, eps, xn, lm_head,

@@ -4,13 +4,15 @@
 //
 // k_head_norm: one workgroup per row, xn = bf16(w * bf16(x * inv)) with
 //   inv = 1 / sqrt(mean(x^2) + eps), the squares summed in double.
-// k_head_gemv: logits[b][v] = bf16(sum_k xn[b][k] W[v][k]) with float accumulation. A
-//   workgroup owns 128 vocabulary rows (four waves of two 16-row tiles) over the whole of K,
-//   so the 1,187 workgroups of V = 151,936 each stream 1.3 MB of weights once, and the
-//   weight matrix is read exactly once per call whatever the batch. The batch is the
-//   MFMA's N side (16 rows per tile, up to four tiles), read from the L2-resident xn.
+// k_head_split (up to 16 rows, and more on small vocabularies), k_head_gemv (the others):
+//   logits[b][v] = bf16(sum_k xn[b][k] W[v][k]) with float accumulation. The weight matrix
+//   is read exactly once per call whatever the batch, which is the MFMA's N side (16 rows
+//   per tile, up to four tiles). k_head_split: a workgroup owns 32 or 64 vocabulary rows and
+//   its waves split K; the batch operand comes from the L2-resident xn. k_head_gemv: a
+//   workgroup owns 128 vocabulary rows, each wave two 16-row tiles over the whole of K,
+//   and the workgroup stages xn in LDS.
 //   For a greedy pick (strim_head_greedy) its epilogue also writes each batch row's first
-//   maximum over the workgroup's 128 logits (as bf16 values, as the sampler reads them),
+//   maximum over the workgroup's logits (as bf16 values, as the sampler reads them),
 //   and the logits may be left unwritten.
 // k_head_pick: one workgroup per batch row merges the rows' tile maxima into the first
 //   maximum of the row: the greedy token, with the sampler's statuses (a NaN or +inf logit:
@@ -91,9 +93,6 @@ __global__ __launch_bounds__(HN_T) void k_head_norm(const uint16_t* x, int64_t x
   }
 }
 
-// NT: 16-row batch tiles (B <= 16 NT). VO: 8-byte logit stores (rows 4-element aligned).
-// MT: 16-row vocabulary tiles per wave; NW: waves per workgroup; NTL: weights loaded
-// nontemporal (streamed once, kept out of the caches that hold xn).
 // The larger of two (value, id) pairs, the smaller id on equal values (NaN never taken).
 __device__ __forceinline__ void hb_take(float& v, int& i, float v2, int i2) {
   if (v2 > v || (v2 == v && i2 < i)) {
@@ -102,9 +101,24 @@ __device__ __forceinline__ void hb_take(float& v, int& i, float v2, int i2) {
   }
 }
 
+// Four logits of one batch row, vocabulary ids vb .. vb + 3 (those below V).
+template <bool VO>
+__device__ __forceinline__ void head_store4(uint16_t* dst, const uint16_t* o, int vb, int V) {
+  if (VO && vb + 3 < V) {
+    *(uint2*)dst = make_uint2((uint32_t)o[0] | ((uint32_t)o[1] << 16),
+                              (uint32_t)o[2] | ((uint32_t)o[3] << 16));
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (vb + i < V) dst[i] = o[i];
+  }
+}
+
+// NT: 16-row batch tiles (B <= 16 NT). VO: 8-byte logit stores (rows 4-element aligned).
 // TB: write the tile maxima to tbest[n][blockIdx.x] = {value bits (NaN: the tile holds a
-// NaN or +inf), id}; out NULL: no logits stored.
-template <int NT, bool VO, bool TB = false, int MT = HG_MT, int NW = HG_W, bool NTL = false>
+// NaN or +inf), id}; out NULL: no logits stored. MT: 16-row vocabulary tiles per wave; NW:
+// waves per workgroup.
+template <int NT, bool VO, bool TB, int MT, int NW>
 __global__ __launch_bounds__(NW* WAVE) void k_head_gemv(const uint16_t* xn, int64_t xn_stride,
                                                           int B, int K, const uint16_t* W,
                                                           int64_t w_stride, int V,
@@ -115,16 +129,10 @@ __global__ __launch_bounds__(NW* WAVE) void k_head_gemv(const uint16_t* xn, int6
   const int v0 = blockIdx.x * (NW * MT * 16) + wv * (MT * 16);
   // rows past V or B read a clamped row; their results are not stored
   const uint16_t* arow[MT];
-  const uint16_t* brow[NT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     const int v = min(v0 + mt * 16 + r16, V - 1);
     arow[mt] = W + (int64_t)v * w_stride + 8 * h;
-  }
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    const int n = min(nt * 16 + r16, B - 1);
-    brow[nt] = xn + (int64_t)n * xn_stride + 8 * h;
   }
   f32x4_t acc[MT][NT];
 #pragma unroll
@@ -132,126 +140,90 @@ __global__ __launch_bounds__(NW* WAVE) void k_head_gemv(const uint16_t* xn, int6
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   // two register buffers: the next step's loads are in flight while this step multiplies
-  uint4 a[2][MT][4], bq[2][NT][4];
+  uint4 a[2][MT][4];
   auto loada = [&](int buf, int kb) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const u32x4_t* src = (const u32x4_t*)(arow[mt] + kb + 32 * q);
-        const u32x4_t v = NTL ? __builtin_nontemporal_load(src) : *src;
-        a[buf][mt][q] = make_uint4(v[0], v[1], v[2], v[3]);
-      }
-  };
-  auto load = [&](int buf, int kb) {
-    loada(buf, kb);
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) bq[buf][nt][q] = *(const uint4*)(brow[nt] + kb + 32 * q);
-  };
-  auto mma = [&](int buf) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
-          acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              __builtin_bit_cast(bf16x8_t, a[buf][mt][q]),
-              __builtin_bit_cast(bf16x8_t, bq[buf][nt][q]), acc[mt][nt], 0, 0, 0);
+      for (int q = 0; q < 4; ++q) a[buf][mt][q] = *(const uint4*)(arow[mt] + kb + 32 * q);
   };
   // K is a multiple of 2 steps (the host checks), so every load and multiply is
   // unconditional (the last prefetch reloads the last step and is not used), and the
   // scheduling barriers keep each buffer's loads issued before the other buffer's
   // multiplies: left alone, the compiler sinks the loads next to their use
   const int nsteps = K / HG_KS;
-  if constexpr (NT == 1) {
-    load(0, 0);
-    for (int s = 0; s < nsteps; s += 2) {
-      load(1, (s + 1) * HG_KS);
-      __builtin_amdgcn_sched_barrier(0);
-      mma(0);
-      __builtin_amdgcn_sched_barrier(0);
-      load(0, min(s + 2, nsteps - 2) * HG_KS);
-      __builtin_amdgcn_sched_barrier(0);
-      mma(1);
-      __builtin_amdgcn_sched_barrier(0);
+  // Several batch tiles: every wave needs the same 16 NT rows of xn at each step, so
+  // the workgroup stages them in LDS once (double-buffered, rows padded by 16 bytes so
+  // the 16 rows a wave reads fall in different banks) instead of each wave reading
+  // them from L2 (four times the bytes: that bound B = 64 at 2.7 TB/s). Thread t
+  // carries NT 16-byte pieces of the next step's slice while this step multiplies.
+  constexpr int XR = 16 * NT, XW = HG_KS + 8;  // rows, padded row length (bf16)
+  __shared__ __attribute__((aligned(16))) uint16_t s_x[2][XR][XW];
+  struct Slice {
+    uint4 v[NT];
+  };
+  auto xload = [&](int kb) -> Slice {
+    Slice xr;
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      const int e = (int)threadIdx.x + NW * WAVE * i;  // piece e: row e / 16, column 8 (e % 16)
+      const int row = e >> 4, col = (e & 15) * 8;
+      const int n = min(row, B - 1);
+      xr.v[i] = *(const uint4*)(xn + (int64_t)n * xn_stride + kb + col);
     }
-  } else {
-    // Several batch tiles: every wave needs the same 16 NT rows of xn at each step, so
-    // the workgroup stages them in LDS once (double-buffered, rows padded by 16 bytes so
-    // the 16 rows a wave reads fall in different banks) instead of each wave reading
-    // them from L2 (four times the bytes: that bound B = 64 at 2.7 TB/s). Thread t
-    // carries NT 16-byte pieces of the next step's slice while this step multiplies.
-    constexpr int XR = 16 * NT, XW = HG_KS + 8;  // rows, padded row length (bf16)
-    __shared__ __attribute__((aligned(16))) uint16_t s_x[2][XR][XW];
-    struct Slice {
-      uint4 v[NT];
-    };
-    auto xload = [&](int kb) -> Slice {
-      Slice xr;
+    return xr;
+  };
+  auto xstore = [&](int buf, const Slice& xr) {
 #pragma unroll
-      for (int i = 0; i < NT; ++i) {
-        const int e = (int)threadIdx.x + NW * WAVE * i;  // piece e: row e / 16, column 8 (e % 16)
-        const int row = e >> 4, col = (e & 15) * 8;
-        const int n = min(row, B - 1);
-        xr.v[i] = *(const uint4*)(xn + (int64_t)n * xn_stride + kb + col);
-      }
-      return xr;
-    };
-    auto xstore = [&](int buf, const Slice& xr) {
+    for (int i = 0; i < NT; ++i) {
+      const int e = (int)threadIdx.x + NW * WAVE * i;
+      *(uint4*)&s_x[buf][e >> 4][(e & 15) * 8] = xr.v[i];
+    }
+  };
+  // the multiplies of one step from LDS buffer buf, the B operand read one K slice (q)
+  // at a time next to its MFMAs: NT registers of it live instead of 4 NT
+  auto mma_lds = [&](int buf, int abuf) {
 #pragma unroll
-      for (int i = 0; i < NT; ++i) {
-        const int e = (int)threadIdx.x + NW * WAVE * i;
-        *(uint4*)&s_x[buf][e >> 4][(e & 15) * 8] = xr.v[i];
-      }
-    };
-    // the multiplies of one step from LDS buffer buf, the B operand read one K slice (q)
-    // at a time next to its MFMAs: NT registers of it live instead of 4 NT
-    auto mma_lds = [&](int buf, int abuf) {
+    for (int q = 0; q < 4; ++q) {
+      uint4 bx[NT];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        uint4 bx[NT];
+      for (int nt = 0; nt < NT; ++nt)
+        bx[nt] = *(const uint4*)&s_x[buf][nt * 16 + r16][32 * q + 8 * h];
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)
-          bx[nt] = *(const uint4*)&s_x[buf][nt * 16 + r16][32 * q + 8 * h];
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-          for (int nt = 0; nt < NT; ++nt)
-            acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                __builtin_bit_cast(bf16x8_t, a[abuf][mt][q]), __builtin_bit_cast(bf16x8_t, bx[nt]),
-                acc[mt][nt], 0, 0, 0);
-      }
-    };
-    static_assert(NT * NW * WAVE * 8 == XR * HG_KS, "one step's slice: NT pieces a thread");
-    // The barrier waits for the LDS stores alone: __syncthreads' fence would also wait
-    // for the next step's weight loads, the prefetch this loop depends on. The slice's
-    // loads are issued before the weights', so its store waits for them only.
-    auto sync_lds = []() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-    // Unrolled by two so each register buffer has a fixed index (the host checks that K
-    // is a multiple of two steps; the last prefetch reloads the last step, unused).
-    xstore(0, xload(0));
-    loada(0, 0);
-    sync_lds();
-    for (int s = 0; s < nsteps; s += 2) {
-      const Slice x1 = xload((s + 1) * HG_KS);
-      loada(1, (s + 1) * HG_KS);
-      __builtin_amdgcn_sched_barrier(0);
-      mma_lds(0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      xstore(1, x1);
-      sync_lds();
-      const int s2 = min(s + 2, nsteps - 2) * HG_KS;
-      const Slice x0 = xload(s2);
-      loada(0, s2);
-      __builtin_amdgcn_sched_barrier(0);
-      mma_lds(1, 1);
-      __builtin_amdgcn_sched_barrier(0);
-      xstore(0, x0);
-      sync_lds();
+          acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              __builtin_bit_cast(bf16x8_t, a[abuf][mt][q]), __builtin_bit_cast(bf16x8_t, bx[nt]),
+              acc[mt][nt], 0, 0, 0);
     }
+  };
+  static_assert(NT * NW * WAVE * 8 == XR * HG_KS, "one step's slice: NT pieces a thread");
+  // The barrier waits for the LDS stores alone: __syncthreads' fence would also wait
+  // for the next step's weight loads, the prefetch this loop depends on. The slice's
+  // loads are issued before the weights', so its store waits for them only.
+  auto sync_lds = []() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+  // Unrolled by two so each register buffer has a fixed index (the host checks that K
+  // is a multiple of two steps; the last prefetch reloads the last step, unused).
+  xstore(0, xload(0));
+  loada(0, 0);
+  sync_lds();
+  for (int s = 0; s < nsteps; s += 2) {
+    const Slice x1 = xload((s + 1) * HG_KS);
+    loada(1, (s + 1) * HG_KS);
+    __builtin_amdgcn_sched_barrier(0);
+    mma_lds(0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    xstore(1, x1);
+    sync_lds();
+    const int s2 = min(s + 2, nsteps - 2) * HG_KS;
+    const Slice x0 = xload(s2);
+    loada(0, s2);
+    __builtin_amdgcn_sched_barrier(0);
+    mma_lds(1, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    xstore(0, x0);
+    sync_lds();
   }
   // lane l holds rows 4 h + i of each tile for batch row nt 16 + r16
   float bv[NT];
@@ -280,14 +252,7 @@ __global__ __launch_bounds__(NW* WAVE) void k_head_gemv(const uint16_t* xn, int6
       }
       if (n >= B || out == nullptr) continue;
       uint16_t* dst = out + (int64_t)n * out_stride + vb;
-      if (VO && vb + 3 < V) {
-        *(uint2*)dst = make_uint2((uint32_t)o[0] | ((uint32_t)o[1] << 16),
-                                  (uint32_t)o[2] | ((uint32_t)o[3] << 16));
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (vb + i < V) dst[i] = o[i];
-      }
+      head_store4<VO>(dst, o, vb, V);
     }
   }
   if constexpr (TB) {
@@ -321,6 +286,144 @@ __global__ __launch_bounds__(NW* WAVE) void k_head_gemv(const uint16_t* xn, int6
         hb_take(v, i, s_v[q][n], s_i[q][n]);
       }
       tbest[(int64_t)n * gridDim.x + blockIdx.x] =
+          make_uint2(__float_as_uint(nan ? __uint_as_float(0x7FC00000u) : v), (uint32_t)i);
+    }
+  }
+}
+
+// The same product with K split over the workgroup's waves: wave w multiplies the steps
+// [w n / NW, (w + 1) n / NW) of the same MT 16-row tiles, and the partial sums are added in
+// wave order through LDS. Bound by HBM. A workgroup that holds 128 rows over the whole of K
+// leaves the chip half empty at its end, or throughout where V / 128 is near or below the
+// 256 CUs; K / NW on 32 rows makes pieces a sixteenth the size (each wave's batch slice
+// is read from L2 either way at one batch tile). B = 8, K = 5,120: 109.6 -> 77.8 us at
+// V = 40,000 (65 at a plain read's 6.26 TB/s), 54.4 -> 21.6 at V = 8,192, 280.0 -> 272.8 at
+// V = 151,936; K = 2,048, V = 151,936: 143.5 -> 109.7.
+template <int NT, bool VO, bool TB, int MT, int NW>
+__global__ __launch_bounds__(NW* WAVE) void k_head_split(const uint16_t* xn, int64_t xn_stride,
+                                                           int B, int K, const uint16_t* W,
+                                                           int64_t w_stride, int V,
+                                                           uint16_t* out, int64_t out_stride,
+                                                           uint2* tbest) {
+  __shared__ f32x4_t s_acc[NW][MT * NT][WAVE];
+  const int lane = threadIdx.x & (WAVE - 1), wv = wave_id();
+  const int h = lane >> 4, r16 = lane & 15;
+  const int v0 = blockIdx.x * (MT * 16);
+  const int nsteps = K / HG_KS, s0 = wv * nsteps / NW, n = (wv + 1) * nsteps / NW - s0;
+  // rows past V or B read a clamped row; their results are not stored
+  const uint16_t* arow[MT];
+  const uint16_t* brow[NT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+    arow[mt] = W + (int64_t)min(v0 + mt * 16 + r16, V - 1) * w_stride + 8 * h + s0 * HG_KS;
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt)
+    brow[nt] = xn + (int64_t)min(nt * 16 + r16, B - 1) * xn_stride + 8 * h + s0 * HG_KS;
+  f32x4_t acc[MT][NT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  uint4 a[2][MT][4], bq[2][NT][4];
+  auto load = [&](int buf, int s) {
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) a[buf][mt][q] = *(const uint4*)(arow[mt] + s * HG_KS + 32 * q);
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) bq[buf][nt][q] = *(const uint4*)(brow[nt] + s * HG_KS + 32 * q);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto mma = [&](int buf) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+          acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              __builtin_bit_cast(bf16x8_t, a[buf][mt][q]),
+              __builtin_bit_cast(bf16x8_t, bq[buf][nt][q]), acc[mt][nt], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // (a wave may have no step when K has fewer than NW; the last one or two steps are peeled,
+  // so that no load in the loop is conditional and none is repeated)
+  if (n > 0) {
+    load(0, 0);
+    int s = 0;
+    for (; s + 2 < n; s += 2) {
+      load(1, s + 1);
+      mma(0);
+      load(0, s + 2);
+      mma(1);
+    }
+    if (s + 2 == n) {
+      load(1, s + 1);
+      mma(0);
+      mma(1);
+    } else {
+      mma(0);
+    }
+  }
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) s_acc[wv][nt * MT + mt][lane] = acc[mt][nt];
+  __syncthreads();
+  __shared__ float s_v[TB ? MT : 1][16 * NT];
+  __shared__ int s_i[TB ? MT : 1][16 * NT];
+  // tile e of wave e % NW; lane l holds rows 4 h + i of it for batch row nt 16 + r16
+#pragma unroll
+  for (int e0 = 0; e0 < MT * NT; e0 += NW) {
+    const int e = e0 + wv;
+    if (e >= MT * NT) break;
+    const int mt = e % MT, nr = e / MT * 16 + r16, vb = v0 + mt * 16 + 4 * h;
+    f32x4_t sum = s_acc[0][e][lane];
+#pragma unroll
+    for (int q = 1; q < NW; ++q) sum += s_acc[q][e][lane];
+    uint16_t o[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = head_bf16(sum[i]);
+    if (nr < B && out != nullptr) head_store4<VO>(out + (int64_t)nr * out_stride + vb, o, vb, V);
+    if constexpr (TB) {
+      float bv = -INFINITY;
+      int bi = INT_MAX;
+      bool bad = false;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (vb + i < V) {
+          const float f = __uint_as_float((uint32_t)o[i] << 16);
+          bad = bad || !(f < INFINITY);  // NaN or +inf
+          hb_take(bv, bi, f, vb + i);
+        }
+#pragma unroll
+      for (int sh = 16; sh < WAVE; sh <<= 1) {
+        const float v2 = __shfl_xor(bv, sh);
+        const int i2 = __shfl_xor(bi, sh);
+        bad = (__shfl_xor((int)bad, sh) != 0) || bad;
+        hb_take(bv, bi, v2, i2);
+      }
+      if (h == 0) {
+        s_v[mt][nr] = bad ? __uint_as_float(0x7FC00000u) : bv;
+        s_i[mt][nr] = bi;
+      }
+    }
+  }
+  if constexpr (TB) {
+    __syncthreads();
+    const int nr = (int)threadIdx.x;
+    if (nr < B && nr < 16 * NT) {
+      float v = s_v[0][nr];
+      int i = s_i[0][nr];
+      bool nan = !(v == v);
+#pragma unroll
+      for (int q = 1; q < MT; ++q) {
+        nan = nan || !(s_v[q][nr] == s_v[q][nr]);
+        hb_take(v, i, s_v[q][nr], s_i[q][nr]);
+      }
+      tbest[(int64_t)nr * gridDim.x + blockIdx.x] =
           make_uint2(__float_as_uint(nan ? __uint_as_float(0x7FC00000u) : v), (uint32_t)i);
     }
   }
@@ -378,35 +481,42 @@ hipError_t launch_head(const void* hidden, int64_t hidden_stride, int B, int K,
     src = (const uint16_t*)xn;
     src_stride = K;
   }
-  // vocabulary rows per workgroup: 4 waves of HG_MT 16-row tiles (one tile a wave above
-  // B = 16 measured slower: 767 against 534 us at B = 64, the staged batch slice is then
-  // loaded for half as many weight rows)
+  // One batch tile: always split. K from 4,096 (four steps and more a wave) over eight
+  // waves, else four (B = 8, V = 151,936: 272.8 against 275.8 us at K = 5,120, 117.5 against
+  // 109.7 at K = 2,048). 64 rows a workgroup, in place of 32, halve the reads of xn, which
+  // count where its tile's rows are distinct and the vocabulary still fills the chip
+  // (K = 5,120, B = 16: 303 against 317 us at V = 151,936, 157 against 169 at 80,000, but
+  // 92.6 against 89.2 at 40,000; B = 8, V = 151,936: 284 against 273).
+  // More tiles: the staged slice of xn is worth more than the split, until its 128-row
+  // workgroups leave most CUs idle (its time hardly falls below V = 20,000, the split's is
+  // in proportion to V. K = 5,120, V = 8,192: B = 24 50.4 -> 26.5 us, B = 64 59.1 -> 37.8;
+  // V = 20,000: B = 24 56.1 against 62.0, B = 64 65 against 97; K = 3,584, V = 10,672:
+  // B = 24 36.9 -> 30.7, B = 64 42.9 against 47.1).
   const int nt = (B + 15) / 16;
-  const int rows = HG_W * HG_MT * 16;
-  const dim3 grid((unsigned)((V + rows - 1) / rows)), blk(HG_W * WAVE);
-#define STRIM_HEAD_GEMV(NT_, MT_)                                                                \
-  if (tbest && vo)                                                                               \
-    hipLaunchKernelGGL((k_head_gemv<NT_, true, true, MT_>), grid, blk, 0, st, src, src_stride, B, \
-                       K, (const uint16_t*)W, w_stride, V, (uint16_t*)out, out_stride, tbest);    \
-  else if (tbest)                                                                                \
-    hipLaunchKernelGGL((k_head_gemv<NT_, false, true, MT_>), grid, blk, 0, st, src, src_stride,   \
-                       B, K, (const uint16_t*)W, w_stride, V, (uint16_t*)out, out_stride, tbest); \
-  else if (vo)                                                                                   \
-    hipLaunchKernelGGL((k_head_gemv<NT_, true, false, MT_>), grid, blk, 0, st, src, src_stride,   \
-                       B, K, (const uint16_t*)W, w_stride, V, (uint16_t*)out, out_stride,         \
-                       nullptr);                                                                 \
-  else                                                                                           \
-    hipLaunchKernelGGL((k_head_gemv<NT_, false, false, MT_>), grid, blk, 0, st, src, src_stride,  \
-                       B, K, (const uint16_t*)W, w_stride, V, (uint16_t*)out, out_stride,         \
-                       nullptr);
-  if (nt == 1) {
-    STRIM_HEAD_GEMV(1, HG_MT)
-  } else if (nt == 2) {
-    STRIM_HEAD_GEMV(2, HG_MT)
-  } else {
-    STRIM_HEAD_GEMV(4, HG_MT)
-  }
-#undef STRIM_HEAD_GEMV
+  const bool split = nt == 1 || V <= (nt == 2 ? 14336 : 9216);
+  const bool deep = nt == 1 && K >= 4096, tall = deep && B >= 12 && V >= 65536;
+  const int rows = split ? (tall ? 64 : 32) : HG_W * HG_MT * 16;
+  const dim3 grid((unsigned)((V + rows - 1) / rows));
+#define STRIM_HEAD_(K_, NT_, MT_, NW_, VO_, TB_)                                              \
+  hipLaunchKernelGGL((K_<NT_, VO_, TB_, MT_, NW_>), grid, dim3(NW_ * WAVE), 0, st, src,       \
+                     src_stride, B, K, (const uint16_t*)W, w_stride, V, (uint16_t*)out,       \
+                     out_stride, tbest)
+#define STRIM_HEAD(K_, NT_, MT_, NW_)                             \
+  do {                                                            \
+    if (tbest && vo) STRIM_HEAD_(K_, NT_, MT_, NW_, true, true);  \
+    else if (tbest) STRIM_HEAD_(K_, NT_, MT_, NW_, false, true);  \
+    else if (vo) STRIM_HEAD_(K_, NT_, MT_, NW_, true, false);     \
+    else STRIM_HEAD_(K_, NT_, MT_, NW_, false, false);            \
+  } while (0)
+  if (tall) STRIM_HEAD(k_head_split, 1, 4, 8);
+  else if (deep) STRIM_HEAD(k_head_split, 1, 2, 8);
+  else if (nt == 1) STRIM_HEAD(k_head_split, 1, 2, 4);
+  else if (nt == 2 && split) STRIM_HEAD(k_head_split, 2, 2, 4);
+  else if (nt == 2) STRIM_HEAD(k_head_gemv, 2, HG_MT, HG_W);
+  else if (split) STRIM_HEAD(k_head_split, 4, 2, 4);
+  else STRIM_HEAD(k_head_gemv, 4, HG_MT, HG_W);
+#undef STRIM_HEAD
+#undef STRIM_HEAD_
   if (tbest)
     hipLaunchKernelGGL(k_head_pick, dim3((unsigned)B), dim3(HP_T), 0, st, tbest, (int)grid.x,
                        out_ids, out_status);

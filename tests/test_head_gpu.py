@@ -54,6 +54,47 @@ def test_head_logits_match_fp64_product(B, K, V):
     check_logits(to_np(out), xn_ref, W, f"B={B} K={K} V={V}")
 
 
+@pytest.mark.parametrize("B,K,V,pad", [(1, 256, 33, 0), (16, 512, 31, 0), (11, 1280, 4099, 1),
+                                       (16, 3840, 65, 0), (16, 4096, 97, 3), (5, 4352, 8192, 0),
+                                       (11, 4096, 65537, 0), (12, 4096, 65535, 0),
+                                       (12, 4096, 65537, 0), (16, 5120, 65600, 1),
+                                       (17, 256, 14336, 0), (32, 768, 14335, 1),
+                                       (17, 256, 14337, 0), (33, 256, 9216, 0), (64, 1280, 9215, 1),
+                                       (33, 256, 9217, 0)])
+def test_head_split_forms(B, K, V, pad):
+    """K split over a workgroup's waves: fewer steps than waves, step counts that the waves do
+    not share evenly, row tiles past the vocabulary, and both sides of each line of the
+    dispatch (32 or 64 rows, four or eight waves, the staged kernel), with aligned and
+    unaligned output rows; then the greedy pick on the same logits."""
+    print(f"[head] split B={B} K={K} V={V}", flush=True)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(B * 1000 + K + V)
+    x = torch.randn(B, K, device="cuda", generator=g).to(torch.bfloat16)
+    W = (0.05 * torch.randn(V, K, device="cuda", generator=g)).to(torch.bfloat16)
+    buf = torch.full((B, V + pad), 7.0, dtype=torch.bfloat16, device="cuda")
+    st = N.lib().strim_head_logits(ctypes.c_void_p(torch.cuda.current_stream().cuda_stream),
+                                   ctypes.c_void_p(x.data_ptr()), K, B, K, None, 1e-6, None,
+                                   ctypes.c_void_p(W.data_ptr()), K, V,
+                                   ctypes.c_void_p(buf.data_ptr()), V + pad)
+    assert st == 0
+    torch.cuda.synchronize()
+    out, xd = buf[:, :V], x.double()
+    for a in range(0, V, 16_384):  # the bound of check_logits, on the device
+        wd = W[a:a + 16_384].double()
+        ref = xd @ wd.T
+        ulp = torch.exp2(torch.floor(torch.log2(ref.abs().clamp_min(1e-30))) - 7)
+        tol = 0.5 * ulp + 1e-6 * (xd.abs() @ wd.abs().T) + 1e-30
+        err = (out[:, a:a + 16_384].double() - ref).abs()
+        assert bool((err <= tol).all()), f"from {a}: {float((err - tol).max()):.3g} past the bound"
+    assert bool((buf[:, V:] == 7.0).all())
+    c = ops.Context(0, max_rows=B, max_vocab=V)
+    ids, st = ops.head_greedy(c, x, W)
+    torch.cuda.synchronize()
+    assert (st.cpu().numpy() == 0).all()
+    np.testing.assert_array_equal(ids.cpu().numpy(), np.argmax(to_np(out), axis=1))
+    c.close()
+
+
 def test_head_logits_no_norm_and_strided_output():
     # hidden already normalised (norm_weight NULL); logits rows at a stride that is not a
     # multiple of 4 (the element-wise store path) inside a larger buffer
