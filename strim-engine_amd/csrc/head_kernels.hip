@@ -486,7 +486,8 @@ hipError_t launch_head(const void* hidden, int64_t hidden_stride, int B, int K,
   // 109.7 at K = 2,048). 64 rows a workgroup, in place of 32, halve the reads of xn, which
   // count where its tile's rows are distinct and the vocabulary still fills the chip
   // (K = 5,120, B = 16: 303 against 317 us at V = 151,936, 157 against 169 at 80,000, but
-  // 92.6 against 89.2 at 40,000; B = 8, V = 151,936: 284 against 273).
+  // 92.6 against 89.2 at 40,000; B = 8, V = 151,936: 284 against 273; B = 11, V = 65,536:
+  // 124.1 against 127.4).
   // More tiles: the staged slice of xn is worth more than the split, until its 128-row
   // workgroups leave most CUs idle (its time hardly falls below V = 20,000, the split's is
   // in proportion to V. K = 5,120, V = 8,192: B = 24 50.4 -> 26.5 us, B = 64 59.1 -> 37.8;
@@ -494,7 +495,7 @@ hipError_t launch_head(const void* hidden, int64_t hidden_stride, int B, int K,
   // B = 24 36.9 -> 30.7, B = 64 42.9 against 47.1).
   const int nt = (B + 15) / 16;
   const bool split = nt == 1 || V <= (nt == 2 ? 14336 : 9216);
-  const bool deep = nt == 1 && K >= 4096, tall = deep && B >= 12 && V >= 65536;
+  const bool deep = nt == 1 && K >= 4096, tall = deep && B >= 11 && V >= 65536;
   const int rows = split ? (tall ? 64 : 32) : HG_W * HG_MT * 16;
   const dim3 grid((unsigned)((V + rows - 1) / rows));
 #define STRIM_HEAD_(K_, NT_, MT_, NW_, VO_, TB_)                                              \
