@@ -1104,9 +1104,11 @@ __attribute__((not_tail_called)) __device__ __noinline__ XOut gfinal_rest(uint64
       __syncthreads();
       const GCmd cmd = uniform_copy(S.cmd);
       if (cmd.op == GOP_FAIL) return false;
-      if (cmd.op == GOP_SKIP) continue;
-      if (cmd.op == GOP_BOUND) {
-        bound = cmd.bmp;
+      if (cmd.op == GOP_SKIP || cmd.op == GOP_BOUND) {
+        // (a step without a zone has no barrier of its own: every wave has read the
+        // command before the leader posts the next)
+        __syncthreads();
+        if (cmd.op == GOP_BOUND) bound = cmd.bmp;
         continue;
       }
       const int bz = cmd.bz;

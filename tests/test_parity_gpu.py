@@ -351,6 +351,26 @@ def test_wide_nuclei_window_lists(V, B, dtype):
     c.close()
 
 
+@pytest.mark.parametrize("V", [9001, 40001])
+@pytest.mark.parametrize("mode", [O.NOISE_ICDF, O.NOISE_GUMBEL])
+def test_general_steps_without_a_zone(ctx, V, mode):
+    """General rows whose workgroup takes steps that load no zone before one that does: a
+    top-k above the allowed tokens (skipped), a min-p that every allowed token passes (its
+    bound alone is set), both in turn, then a top-p cut in a crowded bin. Each such step is
+    followed at once by the next one's command."""
+    rng = np.random.default_rng(V + mode)
+    B = 8
+    x = np.clip(rng.normal(0, 1.0, size=(B, V)), -4.0, 4.0).astype(np.float32)
+    allowed = rng.random((B, V)) < 0.9
+    p = O.make_params(B, top_k=np.resize([V - 1, V - 1, 0, 0], B),
+                      min_p=np.resize([1e-30, 0.0, 1e-30, 1e-6], B),
+                      top_p=np.resize([0.95, 0.9, 0.5, 0.95, 0.95, 0.02, 0.9, 1.0], B),
+                      seed=rng.integers(0, 2**63, size=B, dtype=np.uint64), position=11)
+    say(f"steps without a zone V={V} mode={mode}")
+    check_sample(ctx, x, p, "bf16", mask=W.pack_mask(allowed), noise_mode=mode,
+                 label=f"steps without a zone V={V}")
+
+
 @pytest.mark.parametrize("V,H", [(5000, 0), (151936, 64), (163841, 0), (248320, 64), (262144, 0)])
 @pytest.mark.parametrize("injected", [False, True])
 def test_rank_noise_candidates(V, H, injected):
