@@ -128,7 +128,8 @@ struct GFinalShared {
   double d[GW];
   uint64_t u[GW], u2[2 * GW];
   int ii[GW];
-  int misc[8];                    // 0 rowfull, 1 rowwin, 2 collect count, 3 some tail
+  int misc[8];                    // 0 rowfull, 1 rowwin, 2 collect count, 3 some tail, 4 token,
+                                  // 5 the leader's verdict, 6 a crowded bin (rank noise)
   uint64_t res[2][4];             // a pick: key, count before, mass before, mass (two
   int32_t tag[2];                 // slots, alternating; tag = the pick's number)
   int zpo[2][LW], zpc[2][LW], zpz[2][LW];  // a zone's parts per chunk: first
@@ -526,8 +527,13 @@ __device__ __noinline__ uint32_t minp_last_fkey(float m, double lmp) {
 // (-1: none kept but the draft). by_rank: a token's noise is that of its rank in the
 // row's order. The entries are first laid out by row bin (each bin's first place from the
 // row's cumulative counts, a token's place in its bin by an atomic), and a token's rank is its
-// bin's first place plus the smaller keys of its bin, so a nucleus of a few thousand
-// tokens needs no sort; past ZCAP entries: -2, the exact resolution.
+// bin's first place plus the smaller keys of its bin. Where a bin holds more than RANK_BIN
+// keys (tied values) that count grows with the square of its keys, and the entries are
+// sorted instead. B = 1, V = 151,936, top-p 0.95, tied tokens at the top: 500 of them take
+// 37.6 us a call (by counts; 56.2 with one read in flight), 1,000 44.9 (sorted; 138.7 by
+// counts), 4,000 89.4 (sorted; 1,754), where the exact resolution takes 450, 473 and 622.
+// Past ZCAP entries: -2, the exact resolution.
+constexpr int RANK_BIN = 512;
 template <int LW>
 __attribute__((not_tail_called)) __device__ __noinline__ int gumbel_kept(
     uint64_t kargs, int r, lds_t<GFinalShared<LW>>* Sl, lds_t<GBig<LW>>* Gl, int bb,
@@ -545,8 +551,9 @@ __attribute__((not_tail_called)) __device__ __noinline__ int gumbel_kept(
   const bool by_rank = (p.flags & STRIM_FLAG_NOISE_BY_RANK) && topp;
   GFinalShared<LW>& S = *(GFinalShared<LW>*)Sl;
   GBig<LW>& G = *(GBig<LW>*)Gl;
-  __syncthreads();  // (the last pick's reads of its state)
   const int t = threadIdx.x, lane = t & (WAVE - 1), w = wave_id();
+  if (t == 0) S.misc[6] = 0;
+  __syncthreads();  // (the last pick's reads of its state)
   if (w == 0) {
     // lane c: chunk c's entries up to its part of the bound's bin
     int lim = 0;
@@ -559,7 +566,10 @@ __attribute__((not_tail_called)) __device__ __noinline__ int gumbel_kept(
     if (lane == W - 1) S.zoff[W] = zof + lim;
   }
   if (by_rank && t < NBW) S.prk[t] = 0u;
+  const bool wide = by_rank && t <= bb && (int)(S.rc[t] - (t > 0 ? S.rc[t - 1] : 0u)) > RANK_BIN;
+  if (__ballot(wide) != 0ull && lane == 0) S.misc[6] = 1;
   __syncthreads();
+  const bool sorted = S.misc[6] != 0;
   const int N = S.zoff[W];
   if (by_rank && N > ZCAP) return -2;
   const bool no_lse = (p.flags & STRIM_FLAG_SCORE_NO_LSE) != 0;
@@ -597,14 +607,26 @@ __attribute__((not_tail_called)) __device__ __noinline__ int gumbel_kept(
   }
   if (by_rank) {
     __syncthreads();
+    if (sorted) bitonic_sort_lds<GT>(G.z.zkey, N);
     for (int i = t; i < N; i += GT) {
       const uint64_t k = G.z.zkey[i];
       if (k > bound) continue;
       const float l = key_l(k);
-      const int bq = row_bin(arow, l);
-      const int z0 = bq > 0 ? (int)S.rc[bq - 1] : 0, z1 = z0 + (int)S.prk[bq];
-      int rank = z0;
-      for (int q = z0; q < z1; ++q) rank += G.z.zkey[q] < k ? 1 : 0;
+      int rank = i;
+      if (!sorted) {
+        const int bq = row_bin(arow, l);
+        const int z0 = bq > 0 ? (int)S.rc[bq - 1] : 0, z1 = z0 + (int)S.prk[bq];
+        rank = z0;
+        int q = z0;
+        for (; q + 8 <= z1; q += 8) {  // (eight reads in flight)
+          uint64_t kq[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) kq[e] = G.z.zkey[q + e];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) rank += kq[e] < k ? 1 : 0;
+        }
+        for (; q < z1; ++q) rank += G.z.zkey[q] < k ? 1 : 0;
+      }
       const float u = noise ? noise[rank] : philox_uniform(pkey, (uint64_t)rank);
       const double sc = (no_lse ? (double)l : ((double)l - (double)m) - lse) + gumbel64(u);
       if (bid < 0 || sc > bsc || (sc == bsc && k < btk)) {

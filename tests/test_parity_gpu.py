@@ -371,6 +371,28 @@ def test_general_steps_without_a_zone(ctx, V, mode):
                  label=f"steps without a zone V={V}")
 
 
+@pytest.mark.parametrize("V", [40001, 151936, 248320])
+@pytest.mark.parametrize("n", [511, 512, 513, 2048, 2049, 4000])
+def test_rank_noise_crowded_bins(V, n):
+    """Rank-indexed Gumbel noise where one bin holds n of the kept tokens, all tied or of a
+    few values, either side of the size from which the kept tokens are sorted; the largest
+    fill the zone (and, at few chunks, overflow the slots: the exact resolution)."""
+    rng = np.random.default_rng(V + n)
+    B = 4
+    x = rng.normal(-12.0, 1.0, size=(B, V)).astype(np.float32)
+    for r in range(B):
+        top = rng.choice(V, size=n, replace=False)
+        x[r, top] = 4.0 if r % 2 == 0 else 4.0 + rng.integers(0, 3, size=n) / 64
+        x[r, rng.choice(V, size=40, replace=False)] = 5.0  # (bins before the crowded one)
+    p = O.make_params(B, top_p=[0.95, 0.9, 0.6, 0.99], flags=[7, 2, 3, 7], position=3,
+                      seed=rng.integers(0, 2**63, size=B, dtype=np.uint64))
+    c = ops.Context(0, max_rows=B, max_vocab=V)
+    say(f"rank noise crowded V={V} n={n}")
+    check_sample(c, x, p, "bf16", noise_mode=O.NOISE_GUMBEL,
+                 noise=rng.random((B, V + 1), dtype=np.float32), label=f"rank crowded n={n}")
+    c.close()
+
+
 @pytest.mark.parametrize("V,H", [(5000, 0), (151936, 64), (163841, 0), (248320, 64), (262144, 0)])
 @pytest.mark.parametrize("injected", [False, True])
 def test_rank_noise_candidates(V, H, injected):
