@@ -963,6 +963,8 @@ __attribute__((not_tail_called)) __device__ __noinline__ XOut gfinal_rest(uint64
     const bool topp = p.top_p < 1.0f;
     const bool minp = p.min_p > 0.0f;
     const bool icdf = a.noise_mode == STRIM_NOISE_ICDF;
+    const bool by_rank = !icdf && (p.flags & STRIM_FLAG_NOISE_BY_RANK) && topp;
+    const int glast = icdf ? -1 : (topp ? 2 : (minp ? 1 : 0));  // a Gumbel row's last filter
     bool pfok = true;  // the prefetched candidates are in LDS
     // (leader) the row bins whose tokens the slots or the window lists hold, read once a
     // bin past the slots is asked for
@@ -1073,7 +1075,11 @@ __attribute__((not_tail_called)) __device__ __noinline__ XOut gfinal_rest(uint64
               if (blo == bhi && blo <= bz) cmd.also = blo;
             }
           }
-          if (bz >= rowwin) {
+          // (a Gumbel draw reads every kept token from the slots: it fails as soon as the
+          // row's last filter ends past them, or a kept set ranked for its noise outgrows
+          // the zone)
+          if (bz >= rowwin ||
+              (step == glast && (bz >= rowfull || (by_rank && rcum.cnt(bz) > (uint64_t)ZCAP)))) {
             cmd.op = GOP_FAIL;
           } else if (zb[0] != bz && zb[1] != bz) {
             int full = rowfull;
@@ -1335,14 +1341,19 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
   int b, j;
   row_bj(a, r, b, j);
   const int t = threadIdx.x, lane = t & (WAVE - 1), w = wave_id();
-  const int V = a.V, W = pre_W;
+  const int W = pre_W;
+  // (kept in scalar registers: read again where they are used, each costs the leader a
+  // round trip to the argument block)
+  int V = a.V, noise_mode = a.noise_mode;
+  const float* noise = a.noise;
+  asm volatile("" : "+s"(V), "+s"(noise_mode), "+s"(noise));
   // ---- every load that does not depend on the row's parameters ------------------
   // the chunk statistics (above), the noise, the draft and the chunks' lattice words (no
   // branch between the loads: a missing optional input reads the row's own state and is
   // ignored; words past a chunk's written bins are dropped later)
   RowState* rsp = &a.s.rs[r];
-  const bool gum = a.noise && a.noise_mode != STRIM_NOISE_ICDF;
-  const float* nz = a.noise ? a.noise + (int64_t)r * a.noise_stride : (const float*)rsp;
+  const bool gum = noise && noise_mode != STRIM_NOISE_ICDF;
+  const float* nz = noise ? noise + (int64_t)r * a.noise_stride : (const float*)rsp;
   const float n0 = nz[gum ? V : 0], n1 = nz[gum ? V : 1];
   const bool vdr = a.verify && j < a.k;
   const int32_t* dp = vdr ? a.drafts + (int64_t)b * a.k + j : (const int32_t*)rsp;
@@ -1371,8 +1382,11 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
     for (int q = 0; q < KP; ++q) {
       const int blk = min(w - 1 + DW * q, npb - 1);
       const int e = blk * 128 + 2 * lane;  // its candidates e, e + 1 (PF even)
-      const int c = e / PF, pl = e - c * PF;
-      const Cand* src = c < wl ? slots + (int64_t)c * SLOT + pl : slots;
+      // (chunk c's place e - c PF, at c SLOT; a 24-bit product: the 64-bit multiply-add the
+      // compiler made of it reads a register that an outstanding load may own, and a wait
+      // for every load then stood between these)
+      const int c = e / PF;
+      const Cand* src = slots + (c < wl ? e + __mul24(c, SLOT - PF) : 0);
       __builtin_amdgcn_global_load_lds((const void*)src,
                                        (lds_t<void>*)((char*)P.pfb + blk * 1024), 16, 0, 0);
     }
@@ -1381,12 +1395,12 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
   // the row's own uniforms (rows without given noise), computed while the loads above
   // are in flight: they depend on the parameters alone
   float pu_draw = 0.0f, pu_acc = 0.0f;
-  if (!a.noise) {
+  if (!noise) {
     const uint64_t pkey = mix64(p.seed, p.position);
     pu_draw = philox_uniform(pkey, 0);
-    pu_acc = philox_uniform(pkey, a.noise_mode == STRIM_NOISE_GUMBEL ? (uint64_t)V : 1u);
+    pu_acc = philox_uniform(pkey, noise_mode == STRIM_NOISE_GUMBEL ? (uint64_t)V : 1u);
   }
-  if (!gfinal_row(a.p[b], V, a.noise_mode, a.dlog != nullptr && vdr)) {
+  if (!gfinal_row(a.p[b], V, noise_mode, a.dlog != nullptr && vdr)) {
     __builtin_amdgcn_s_waitcnt(0);  // (no LDS write may land after the workgroup ends)
     return;
   }
@@ -1444,8 +1458,8 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
     return;
   }
   float u_draw = 0.0f, u_acc = 0.0f;
-  if (a.noise) {
-    if (a.noise_mode == STRIM_NOISE_ICDF) u_draw = n0;
+  if (noise) {
+    if (noise_mode == STRIM_NOISE_ICDF) u_draw = n0;
     u_acc = n1;
   } else {
     u_draw = pu_draw;
@@ -1554,7 +1568,7 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
     const bool topk = p.top_k > 0 && p.top_k < V;
     const bool topp = p.top_p < 1.0f;
     const bool minp = p.min_p > 0.0f;
-    const bool icdf = a.noise_mode == STRIM_NOISE_ICDF;
+    const bool icdf = noise_mode == STRIM_NOISE_ICDF;
 
     // ---- the leader alone ------------------------------------------------------------
     // A row whose zones are small (the common case) is decided by wave 0 alone, with no
@@ -1562,16 +1576,18 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
     // chunks' slot regions (each place's source recorded by its chunk's lane, then the keys
     // and masses built by all lanes) and picks within the wave: up to 64 keys by ranks (one
     // key a lane, the zone read as LDS broadcasts), up to SOLO by a radix select in the
-    // wave. A zone past the slots, or of more than SOLO keys, and Gumbel draws, go to
-    // gfinal_rest's cooperative loop (every wave; it starts over). Both follow the same
-    // decision rules.
+    // wave. A zone past the slots, or of more than SOLO keys, goes to gfinal_rest's
+    // cooperative loop (every wave; it starts over). Both follow the same decision rules.
+    // Gumbel rows: the leader decides the kept set, and every wave scores it (B = 8,
+    // V = 151,936, top-p 0.95, noise by id: 21.8 us a call; 26.7 with the kept set decided
+    // by gfinal_rest too, whose call costs 1.5 us and whose steps have barriers).
     constexpr int SQ = 3, SOLO = SQ * WAVE;  // zone keys a lane holds, a zone's keys
     // (a zone of at most 64 keys starts below 2 SOLO; its rank loop reads up to 7 places
     // past its end)
     static_assert(2 * SOLO + WAVE + 8 <= ZCAP && WAVE + 8 <= GT, "rank loop reads in bounds");
+    const bool by_rank = !icdf && (p.flags & STRIM_FLAG_NOISE_BY_RANK) && topp;
     auto solo = [&](const RowCum& rcum, const GTotals& tt) -> int {  // 0 decided, 1
-      // cooperative, 2 exact resolution
-      if (!icdf) return 1;
+      // cooperative, 2 exact resolution, 3 kept set decided (its Gumbel draw is left)
       const int rowwin = tt.rowwin, rowfull = tt.rowfull, n_all = tt.n_all;
       const bool anytail = tt.anytail != 0;
       const uint64_t S0 = tt.S0;
@@ -1581,9 +1597,11 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
       const int dme = own && cs.n > 0 ? (int)(arow - floorf(cs.m * (float)LBS)) : NOBIN;
       const int nbme = own && cs.n > 0 ? (int)cs.ncand2 : 0;
       // bins {bz, also} into the zone (bz at 0, also after it): 0 loaded, else a verdict
-      auto load = [&](int bz, int also) -> int {
+      // (last: the row's last filter. A Gumbel draw reads every kept token from the slots,
+      // so a kept set that ends past them is the exact resolution's)
+      auto load = [&](int bz, int also, bool last) -> int {
         if (bz >= rowwin) return 2;
-        if (bz >= rowfull) return 1;
+        if (bz >= rowfull) return last && !icdf ? 2 : 1;
         const uint64_t cr = rcum.cnt(bz) - rcum.cnt(bz - 1);
         if (cr > (uint64_t)SOLO) return 1;
         const bool two = also >= 0 && also != bz && also < rowfull &&
@@ -1825,7 +1843,7 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
         const double thr = (double)(p.top_k - 1);
         const int bz = rcum.find(false, thr, rowwin, 0ull, NOBIN);
         if (bz >= rowwin) return 2;
-        if ((v = load(bz, -1)) != 0) return v;
+        if ((v = load(bz, -1, !minp && !topp)) != 0) return v;
         const GHit g = wpick(0, zn0, false, thr, ~0ull, -1, rcum.cnt(bz - 1), rcum.mass(bz - 1));
         if (g.key == ~0ull) return 2;
         if (p.flags & STRIM_FLAG_TOPK_KEEP_TIES) {
@@ -1849,7 +1867,7 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
           } else {
             where(bz, z0, n);
             if (z0 < 0) {
-              if ((v = load(bz, -1)) != 0) return v;
+              if ((v = load(bz, -1, !topp)) != 0) return v;
               z0 = 0;
               n = zn0;
             }
@@ -1872,12 +1890,12 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
         where(bz, z0, n);
         if (z0 < 0) {
           int also = -1;
-          if (!vdr) {
+          if (!vdr && icdf) {
             const int blo = rcum.find(true, (double)u_draw * (double)rcum.mass(bz - 1), bz + 1, 0ull, NOBIN);
             const int bhi = rcum.find(true, (double)u_draw * (double)rcum.mass(bz), bz + 1, 0ull, NOBIN);
             if (blo == bhi && blo <= bz) also = blo;
           }
-          if ((v = load(bz, also)) != 0) return v;
+          if ((v = load(bz, also, true)) != 0) return v;
           z0 = 0;
           n = zn0;
         }
@@ -1897,6 +1915,16 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
         wd = rmass(l_draft, m);
         xb = row_bin(arow, l_draft);
       }
+      if (__builtin_expect(!icdf, 0)) {
+        if (bb1 >= rowfull || (by_rank && rcum.cnt(bb1) > (uint64_t)ZCAP)) return 2;
+        if (lane == 0) {  // (S.res and S.tag: idle until a cooperative pick)
+          S.res[0][0] = bound1;
+          S.res[0][1] = S1;
+          S.res[0][2] = wd;
+          S.tag[0] = bb1;
+        }
+        return 3;
+      }
       // the icdf draw over the kept keys without the draft
       int token;
       if (S1 <= wd) {
@@ -1911,7 +1939,7 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
         }
         where(bz, z0, n);
         if (z0 < 0) {
-          if ((v = load(bz, -1)) != 0) return v;
+          if ((v = load(bz, -1, true)) != 0) return v;
           z0 = 0;
           n = zn0;
         }
@@ -1929,7 +1957,7 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
       RowCum rcum = row_cum<LW>(S, arow, m);
       const GTotals tt = row_totals<LW>(S, W);
       const int verdict = solo(rcum, tt);
-      if (verdict == 1) {
+      if (verdict == 1 || (verdict == 3 && by_rank)) {
 #pragma unroll
         for (int q = 0; q < LPL; ++q) {
           S.rc[LPL * lane + q] = rcum.cq(q);
@@ -1943,7 +1971,19 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
     return uniform_copy(S.misc[5]);
   };
   const int verdict = lat ? decide() : 2;
-  if (verdict == 0) return;
+  if (__builtin_expect(verdict == 0, 1)) return;
+  if (verdict == 3) {
+    // the Gumbel draw over the kept set that the leader decided
+    const uint64_t bound = uniform_copy(S.res[0][0]), S1 = uniform_copy(S.res[0][1]);
+    const uint64_t wd = uniform_copy(S.res[0][2]);
+    const int token =
+        gumbel_kept<LW>(kernel_args(), r, (lds_t<GFinalShared<LW>>*)&S, (lds_t<GBig<LW>>*)&G,
+                        uniform_copy(S.tag[0]), bound, draft, m, S1);
+    // (-1: only the draft kept)
+    finish(STRIM_OK, token < 0 ? arg : token,
+           vdr && (double)u_acc < (double)wd / (double)S1 ? 1 : 0, (double)S1 / RFIX, bound);
+    return;
+  }
   GRow g;
   g.m = m;
   g.l_draft = l_draft;

@@ -371,6 +371,40 @@ def test_general_steps_without_a_zone(ctx, V, mode):
                  label=f"steps without a zone V={V}")
 
 
+@pytest.mark.parametrize("V", [9001, 151936, 200003])
+@pytest.mark.parametrize("n", [1, 64, 65, 192, 193, 3000])
+def test_gumbel_kept_set_edges(V, n):
+    """Gumbel rows of the general class whose cut falls among n tied tokens: either side of
+    the sizes that the leader wave ranks, selects and leaves to the workgroup, and past the
+    slots (the exact resolution). Each filter as the last one, ties kept or not, noise by id
+    and by rank; verify rows with the draft kept, dropped, and the only token kept."""
+    rng = np.random.default_rng(V + n)
+    n = min(n, V // 4)
+    B, k = 8, 2
+    x = rng.normal(-6.0, 1.0, size=(B, k + 1, V)).astype(np.float32)
+    for b in range(B):
+        for j in range(k + 1):
+            top = rng.choice(V, size=n + 30, replace=False)
+            x[b, j, top[:n]] = 3.0
+            x[b, j, top[n:]] = rng.normal(4.0, 0.3, size=30)
+    p = O.make_params(B, top_k=np.resize([0, 30 + (n + 1) // 2, 300, 0], B),
+                      top_p=np.resize([0.7, 1.0, 0.9, 0.95, 0.5], B),
+                      min_p=np.resize([0.0, 0.0, 0.0, 1e-4], B),
+                      flags=np.resize([0, 1, 2, 7, 5], B), position=5,
+                      seed=rng.integers(0, 2**63, size=B, dtype=np.uint64))
+    drafts = x[:, :k].argmax(-1).astype(np.int32)
+    drafts[1::3] = rng.integers(0, V, size=drafts[1::3].shape)
+    x[7, 0, drafts[7, 0]] = 40.0  # (the draft holds everything)
+    c = ops.Context(0, max_rows=B * (k + 1), max_vocab=V)
+    noise = rng.random((B, k + 1, V + 1), dtype=np.float32)
+    say(f"gumbel kept sets V={V} n={n}")
+    check_sample(c, x[:, 0], p, "bf16", noise_mode=O.NOISE_GUMBEL,
+                 noise=np.ascontiguousarray(noise[:, 0]), label=f"gumbel kept V={V} n={n}")
+    check_verify(c, x, k, drafts, p, "bf16", noise_mode=O.NOISE_GUMBEL, noise=noise,
+                 label=f"gumbel kept verify V={V} n={n}")
+    c.close()
+
+
 @pytest.mark.parametrize("V", [40001, 151936, 248320])
 @pytest.mark.parametrize("n", [511, 512, 513, 2048, 2049, 4000])
 def test_rank_noise_crowded_bins(V, n):
