@@ -134,7 +134,8 @@ struct GFinalShared {
   int32_t tag[2];                 // slots, alternating; tag = the pick's number)
   int zpo[2][LW], zpc[2][LW], zpz[2][LW];  // a zone's parts per chunk: first
                                                     // slot, count, place in the zone
-  uint8_t lst[LW];                // per chunk: 1 its window list is written
+  uint8_t lst[LW], nfl[LW];       // per chunk: the bins its window list holds (0: no list),
+                                  // the bins its slots hold (for the cooperative decisions)
   GCmd cmd;                       // the decision loop's current step
   GTotals tot;                    // for the cooperative decisions, with rc and rm cumulative
   uint32_t prk[GT];               // a pick: each zone key's rank and the mass before it
@@ -966,17 +967,15 @@ __attribute__((not_tail_called)) __device__ __noinline__ XOut gfinal_rest(uint64
     const bool by_rank = !icdf && (p.flags & STRIM_FLAG_NOISE_BY_RANK) && topp;
     const int glast = icdf ? -1 : (topp ? 2 : (minp ? 1 : 0));  // a Gumbel row's last filter
     bool pfok = true;  // the prefetched candidates are in LDS
-    // (leader) the row bins whose tokens the slots or the window lists hold, read once a
+    // (leader) the row bins whose tokens the slots or the window lists hold, formed once a
     // bin past the slots is asked for
     int listfull = -1;
     auto lists = [&]() {
       if (listfull >= 0) return;
-      int lim = NBW, has = 0;
+      int lim = NBW;
       if (lane < W) {
-        const ChunkStat& cs = a.s.cstat[(int64_t)r * a.s.wmax + lane];
-        has = a.s.glist != nullptr && r < MAXP && cs.n > 0 && cs.g2 != 0.0f ? 1 : 0;
-        if (cs.n > 0 && !has && cs.ncand < cs.ncand2) lim = min(NBW, S.dch[lane] + (int)cs.ncand);
-        S.lst[lane] = (uint8_t)has;
+        const int held = max((int)S.lst[lane], (int)S.nfl[lane]);
+        if (held < S.nbch[lane]) lim = min(NBW, S.dch[lane] + held);
       }
       lim = wave_min_i(lim);
       listfull = uniform_copy(min(lim, rowwin));
@@ -1341,19 +1340,14 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
   int b, j;
   row_bj(a, r, b, j);
   const int t = threadIdx.x, lane = t & (WAVE - 1), w = wave_id();
-  const int W = pre_W;
-  // (kept in scalar registers: read again where they are used, each costs the leader a
-  // round trip to the argument block)
-  int V = a.V, noise_mode = a.noise_mode;
-  const float* noise = a.noise;
-  asm volatile("" : "+s"(V), "+s"(noise_mode), "+s"(noise));
+  const int V = a.V, W = pre_W;
   // ---- every load that does not depend on the row's parameters ------------------
   // the chunk statistics (above), the noise, the draft and the chunks' lattice words (no
   // branch between the loads: a missing optional input reads the row's own state and is
   // ignored; words past a chunk's written bins are dropped later)
   RowState* rsp = &a.s.rs[r];
-  const bool gum = noise && noise_mode != STRIM_NOISE_ICDF;
-  const float* nz = noise ? noise + (int64_t)r * a.noise_stride : (const float*)rsp;
+  const bool gum = a.noise && a.noise_mode != STRIM_NOISE_ICDF;
+  const float* nz = a.noise ? a.noise + (int64_t)r * a.noise_stride : (const float*)rsp;
   const float n0 = nz[gum ? V : 0], n1 = nz[gum ? V : 1];
   const bool vdr = a.verify && j < a.k;
   const int32_t* dp = vdr ? a.drafts + (int64_t)b * a.k + j : (const int32_t*)rsp;
@@ -1395,12 +1389,12 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
   // the row's own uniforms (rows without given noise), computed while the loads above
   // are in flight: they depend on the parameters alone
   float pu_draw = 0.0f, pu_acc = 0.0f;
-  if (!noise) {
+  if (!a.noise) {
     const uint64_t pkey = mix64(p.seed, p.position);
     pu_draw = philox_uniform(pkey, 0);
-    pu_acc = philox_uniform(pkey, noise_mode == STRIM_NOISE_GUMBEL ? (uint64_t)V : 1u);
+    pu_acc = philox_uniform(pkey, a.noise_mode == STRIM_NOISE_GUMBEL ? (uint64_t)V : 1u);
   }
-  if (!gfinal_row(a.p[b], V, noise_mode, a.dlog != nullptr && vdr)) {
+  if (!gfinal_row(a.p[b], V, a.noise_mode, a.dlog != nullptr && vdr)) {
     __builtin_amdgcn_s_waitcnt(0);  // (no LDS write may land after the workgroup ends)
     return;
   }
@@ -1458,8 +1452,8 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
     return;
   }
   float u_draw = 0.0f, u_acc = 0.0f;
-  if (noise) {
-    if (noise_mode == STRIM_NOISE_ICDF) u_draw = n0;
+  if (a.noise) {
+    if (a.noise_mode == STRIM_NOISE_ICDF) u_draw = n0;
     u_acc = n1;
   } else {
     u_draw = pu_draw;
@@ -1568,7 +1562,7 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
     const bool topk = p.top_k > 0 && p.top_k < V;
     const bool topp = p.top_p < 1.0f;
     const bool minp = p.min_p > 0.0f;
-    const bool icdf = noise_mode == STRIM_NOISE_ICDF;
+    const bool icdf = a.noise_mode == STRIM_NOISE_ICDF;
 
     // ---- the leader alone ------------------------------------------------------------
     // A row whose zones are small (the common case) is decided by wave 0 alone, with no
@@ -1585,7 +1579,6 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
     // (a zone of at most 64 keys starts below 2 SOLO; its rank loop reads up to 7 places
     // past its end)
     static_assert(2 * SOLO + WAVE + 8 <= ZCAP && WAVE + 8 <= GT, "rank loop reads in bounds");
-    const bool by_rank = !icdf && (p.flags & STRIM_FLAG_NOISE_BY_RANK) && topp;
     auto solo = [&](const RowCum& rcum, const GTotals& tt) -> int {  // 0 decided, 1
       // cooperative, 2 exact resolution, 3 kept set decided (its Gumbel draw is left)
       const int rowwin = tt.rowwin, rowfull = tt.rowfull, n_all = tt.n_all;
@@ -1916,6 +1909,7 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
         xb = row_bin(arow, l_draft);
       }
       if (__builtin_expect(!icdf, 0)) {
+        const bool by_rank = (p.flags & STRIM_FLAG_NOISE_BY_RANK) && topp;
         if (bb1 >= rowfull || (by_rank && rcum.cnt(bb1) > (uint64_t)ZCAP)) return 2;
         if (lane == 0) {  // (S.res and S.tag: idle until a cooperative pick)
           S.res[0][0] = bound1;
@@ -1957,13 +1951,17 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
       RowCum rcum = row_cum<LW>(S, arow, m);
       const GTotals tt = row_totals<LW>(S, W);
       const int verdict = solo(rcum, tt);
-      if (verdict == 1 || (verdict == 3 && by_rank)) {
+      if (verdict & 1) {  // (ranked noise reads the counts too)
 #pragma unroll
         for (int q = 0; q < LPL; ++q) {
           S.rc[LPL * lane + q] = rcum.cq(q);
           S.rm[LPL * lane + q] = rcum.mq(q);
         }
         if (lane == 0) S.tot = tt;
+        if (lane < W) {
+          S.lst[lane] = a.s.glist != nullptr && r < MAXP && cs.n > 0 ? (uint8_t)cs.g2 : 0;
+          S.nfl[lane] = (uint8_t)cs.ncand;
+        }
       }
       if (lane == 0) S.misc[5] = verdict;
     }

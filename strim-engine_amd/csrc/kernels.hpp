@@ -68,7 +68,7 @@ struct ChunkStat {
   int32_t arg;     // first id reaching m
   uint32_t ncand;  // fast rows: candidates in the chunk's slot region (> SLOT: overflow);
                    // general rows: window bins whose tokens are all written (nfull)
-  float g2;        // general rows: nonzero when the chunk's window list is written (glist)
+  float g2;        // general rows: the bins its window list holds (glist; 0: no list)
   uint32_t ncand2; // general rows: window bins with lattice words written (nb: the last
                    // non-empty bin + 1); LNONE when the lattice cannot hold the row
   uint32_t pad_;
@@ -145,8 +145,8 @@ struct Scratch {
                                   // chunk, its inclusive count prefix << LCSH | its mass
                                   // (2^37 per unit of exp(l - A / LBS), A the bin's index)
   uint16_t* glist;                // [min(rows, MAXP)][wmax][CHUNK] general rows whose nucleus
-                                  // outgrows the slots: every window token's place in the
-                                  // chunk, in bin order (null: none are written)
+                                  // outgrows the slots: the places in the chunk of the tokens
+                                  // of its first g2 window bins, in bin order (null: none)
   int32_t wmax;
 };
 

@@ -34,8 +34,8 @@ struct StreamShared {
   // general rows: the window's lattice bins (count << LCSH | mass), then each bin's
   // exclusive count prefix (its first entry in the chunk's slot region)
   unsigned long long lat[GEN ? NBW : 1];
-  uint32_t lpre[GEN ? NBW : 1];
-  // a window list being ordered: every window token's place in the chunk, in bin order
+  uint32_t lpre[GEN ? NBW + 1 : 1];
+  // a window list being ordered: its tokens' places in the chunk, in bin order
   __attribute__((aligned(16))) uint16_t wl[GEN ? CHUNK : 8];
   uint32_t lad[2 * WAVE];
   float v[SMAXW];
@@ -585,39 +585,66 @@ __global__ __launch_bounds__(stpb<SSEG>()) void k_stream(const void* pre_logits,
         }
         nfull = wave_sum(nfull);
         nbl = wave_max_i(nbl);
-        // The window list: when the slots do not hold the whole window and the bins they
-        // hold carry less of the chunk's mass than the row keeps, the cut or the draw is
-        // likely below them, and the list lets k_gfinal gather such a bin's tokens from
-        // their logits instead of streaming the whole row for it (a guess only: without
-        // the list the streaming pass decides the same). Rows with penalties have no list:
-        // a token's logit alone does not give its value. The list costs the wide-nucleus
-        // rows' k_stream 1.2 us (8.1 -> 9.3) and saves k_gfinal 38; written for every
-        // general row it would cost the others as much for nothing.
-        int list = 0;
-        if (nfull < nbl && !pen && a.s.glist != nullptr && r < MAXP) {
-          double held = 0.0;
-#pragma unroll
-          for (int q = 0; q < LPL; ++q) {
-            const int bq = LPL * lane + q;
-            const float lb = (atop - (float)bq) * (1.0f / (float)LBS) - m_w;
-            held += bq < nfull ? (double)(hw[q] & LMMASK) * (double)__builtin_amdgcn_exp2f(lb * 1.44269504f)
-                               : 0.0;
-          }
-          held = wave_sum(held) * 0x1p-37;
-          // (without top-p a draw past 95 % of the mass takes the pass: 25 us one time in 20
-          // or fewer, about the list's own cost)
-          const double keep = p.top_p < 1.0f ? (double)p.top_p : 0.95;
-          list = topk || held < keep * cs.S ? 1 : 0;
-        }
 #pragma unroll
         for (int q = 0; q < LPL; ++q)
           if (LPL * lane + q < nbl) lw[LPL * lane + q] = hw[q];
         if (lane == 0) {
           S.i[0] = nfull < nbl ? nfull : nbl;
           S.i[1] = nbl;
-          S.i[2] = list;
         }
-        if (lane == WAVE - 1) S.i[3] = (int)run;
+        if (lane == WAVE - 1) S.lpre[NBW] = run;
+      } else if (w == 1 && !pen) {
+        // The window list: when the row's cut or draw is likely below the bins that the
+        // slots hold, the list lets k_gfinal gather such a bin's tokens from their logits
+        // instead of streaming the whole row for it (a guess only: without the list the
+        // streaming pass decides the same). The guess takes the chunk for a fair share of
+        // the row: a top-k row needs the bins of its first 1.5 k / W tokens, another those
+        // before the kept share of its mass (without top-p 0.95: a draw past it takes the
+        // pass, one time in 20 or fewer), squared: rows whose largest tokens lie in a few
+        // chunks cut above where most chunks alone would. The list ends past twice that
+        // count, or past a quarter of the mass that top-p drops, and four bins; a chunk of few
+        // tokens (the row's last one: no fair share) is listed if anything before that end
+        // is not in its slots. Formed by wave 1 beside wave 0's prefixes. What it costs
+        // k_stream and saves k_gfinal (us): 8 flat rows with top-p 0.95 1.1 and 43; 40 rows
+        // with top-k 400 0.6 (4.3 when every top-k row's window was listed).
+        // No list: rows with penalties (a token's logit alone does not give its value), and
+        // where no decision reads one (a Gumbel draw reads the slots, so only a filter
+        // before the last one may end past them).
+        const bool lists = a.s.glist != nullptr && r < MAXP &&
+                           (a.noise_mode == STRIM_NOISE_ICDF ||
+                            (p.top_p < 1.0f && (topk || p.min_p > 0.0f)));
+        uint32_t val[LPL], sum = 0u, t1, t2;
+        if (topk) {
+#pragma unroll
+          for (int q = 0; q < LPL; ++q) val[q] = (uint32_t)(S.lat[LPL * lane + q] >> LCSH);
+          const uint32_t share = (uint32_t)p.top_k / (uint32_t)P.W;
+          t1 = share + (share >> 1) + 1u;
+          t2 = 2u * share + 32u;
+        } else {
+          const float unit = 0x1p-13f / (float)cs.S;  // 2^24: the chunk's mass
+#pragma unroll
+          for (int q = 0; q < LPL; ++q) {
+            const int bq = LPL * lane + q;
+            const float lb = (atop - (float)bq) * (1.0f / (float)LBS) - m_w;
+            val[q] = (uint32_t)((float)(S.lat[bq] & LMMASK) * unit *
+                                __builtin_amdgcn_exp2f(lb * 1.44269504f));
+          }
+          const float keep = p.top_p < 1.0f ? p.top_p : 0.95f;
+          t2 = p.top_p < 1.0f ? (uint32_t)((0.75f + 0.25f * keep) * 0x1p24f) : ~0u;
+          t1 = cs.n <= CHUNK / 4 ? t2 : (uint32_t)(keep * keep * 0x1p24f);
+        }
+#pragma unroll
+        for (int q = 0; q < LPL; ++q) sum += val[q];
+        sum = wave_incl_scan_u32(sum) - sum;
+        int n1 = 0, n2 = 0;  // the bins before which less than t1, t2 lies
+#pragma unroll
+        for (int q = 0; q < LPL; ++q) {
+          n1 += sum < t1 ? 1 : 0;
+          n2 += sum < t2 ? 1 : 0;
+          sum += val[q];
+        }
+        n1 = wave_sum(n1 | n2 << 16);
+        if (lane == 0) S.i[2] = lists ? n1 : 0;
       }
       __syncthreads();
       const int nfull = S.i[0];
@@ -631,19 +658,21 @@ __global__ __launch_bounds__(stpb<SSEG>()) void k_stream(const void* pre_logits,
           if (lbw[s][e] >= 0 && lbw[s][e] < nfull)
             dst[S.lpre[lbw[s][e]] + lrank[s][e]] = Cand{v[s][e], i0[s] + e};
       cs_ncand = (uint32_t)nfull;
-      cs_ncand2 = (uint32_t)S.i[1];
-      if (S.i[2]) {  // (uniform over the workgroup)
+      const int nbl = S.i[1];
+      cs_ncand2 = (uint32_t)nbl;
+      if (!pen && nfull < nbl && (S.i[2] & 0xFFFF) > nfull) {  // (uniform)
+        const int lend = min((S.i[2] >> 16) + 4, nbl);
 #pragma unroll
         for (int s = 0; s < SSEG; ++s)
 #pragma unroll
           for (int e = 0; e < EPT; ++e)
-            if (lbw[s][e] >= 0)
+            if (lbw[s][e] >= 0 && lbw[s][e] < lend)
               S.wl[S.lpre[lbw[s][e]] + lrank[s][e]] = (uint16_t)(i0[s] + e - c0);
         __syncthreads();
-        const int nw = S.i[3];
+        const int nw = (int)S.lpre[lend];
         uint16_t* gl = a.s.glist + ((int64_t)r * a.s.wmax + c) * CHUNK;
         for (int i = EPT * t; i < nw; i += EPT * STPB) *(uint4*)(gl + i) = *(const uint4*)(S.wl + i);
-        cs.g2 = 1.0f;
+        cs.g2 = (float)lend;
       }
     } else if (!qdraft && !gum_nf) {
       cs_ncand2 = LNONE;  // the lattice cannot hold the row: k_gfinal resolves it exactly

@@ -351,6 +351,40 @@ def test_wide_nuclei_window_lists(V, B, dtype):
     c.close()
 
 
+@pytest.mark.parametrize("V", [9001, 40001, 151936, 248320])
+@pytest.mark.parametrize("mode", [O.NOISE_ICDF, O.NOISE_GUMBEL])
+def test_window_list_ends(V, mode):
+    """Rows whose chunks are unlike each other, so that a cut or a draw falls before, in and
+    past the bins that some chunk's window list holds, beside chunks without a list: chunks
+    shifted against each other, a dominant token in every second chunk, top-k near what the
+    chunks' slots hold together, and filters after the one that reads the lists."""
+    rng = np.random.default_rng(V + mode)
+    B, W = 12, (V + 4095) // 4096
+    x = rng.normal(0, 1.0, size=(B, V)).astype(np.float32)
+    chunk = np.arange(V) // 4096
+    x[1] -= 3.0 * (chunk % 2)
+    x[2] += 0.2 * (chunk % 5)
+    for c in range(0, W, 2):
+        x[3, min(c * 4096 + 7, V - 1)] = 9.0
+        x[4, min(c * 4096 + 9, V - 1)] = 7.0
+    x[5] *= 2.0
+    x[6] = np.round(x[6] * 16) / 16
+    p = O.make_params(B, top_p=np.resize([0.95, 0.9, 0.8, 0.97, 0.9, 0.95, 1.0], B),
+                      top_k=[0, 0, 0, 0, 0, 0, 0, 150 * W, 200 * W, 256 * W, 300 * W, 100 * W],
+                      min_p=np.where(np.arange(B) % 5 == 4, 1e-3, 0.0) * 0.3,
+                      temperature=np.resize([1.0, 0.8], B), position=7,
+                      seed=rng.integers(0, 2**63, size=B, dtype=np.uint64))
+    c = ops.Context(0, max_rows=B, max_vocab=V)
+    for it in range(4):
+        n = V + 1 if mode == O.NOISE_GUMBEL else 2
+        noise = rng.random((B, n), dtype=np.float32)
+        noise[:, 0] = [0.02, 0.4, 0.8, 0.999][it]
+        say(f"window list ends V={V} mode={mode} it={it}")
+        check_sample(c, x, p, "bf16" if it % 2 else "f32", noise_mode=mode, noise=noise,
+                     probs=it == 0, label=f"window list ends V={V}")
+    c.close()
+
+
 @pytest.mark.parametrize("V", [9001, 40001])
 @pytest.mark.parametrize("mode", [O.NOISE_ICDF, O.NOISE_GUMBEL])
 def test_general_steps_without_a_zone(ctx, V, mode):
