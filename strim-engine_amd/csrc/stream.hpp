@@ -599,9 +599,9 @@ __global__ __launch_bounds__(stpb<SSEG>()) void k_stream(const void* pre_logits,
         // instead of streaming the whole row for it (a guess only: without the list the
         // streaming pass decides the same). The guess takes the chunk for a fair share of
         // the row: a top-k row needs the bins of its first 1.5 k / W tokens, another those
-        // before the kept share of its mass (without top-p 0.95: a draw past it takes the
-        // pass, one time in 20 or fewer), squared: rows whose largest tokens lie in a few
-        // chunks cut above where most chunks alone would. The list ends past twice that
+        // before nine tenths of the kept share of its mass (without top-p 0.95: a draw past
+        // it takes the pass, one time in 20 or fewer): rows whose largest tokens lie in a
+        // few chunks cut above where most chunks alone would. The list ends past twice that
         // count, or past a quarter of the mass that top-p drops, and four bins; a chunk of few
         // tokens (the row's last one: no fair share) is listed if anything before that end
         // is not in its slots. Formed by wave 1 beside wave 0's prefixes. What it costs
@@ -631,7 +631,7 @@ __global__ __launch_bounds__(stpb<SSEG>()) void k_stream(const void* pre_logits,
           }
           const float keep = p.top_p < 1.0f ? p.top_p : 0.95f;
           t2 = p.top_p < 1.0f ? (uint32_t)((0.75f + 0.25f * keep) * 0x1p24f) : ~0u;
-          t1 = cs.n <= CHUNK / 4 ? t2 : (uint32_t)(keep * keep * 0x1p24f);
+          t1 = cs.n <= CHUNK / 4 ? t2 : (uint32_t)(0.9f * keep * 0x1p24f);
         }
 #pragma unroll
         for (int q = 0; q < LPL; ++q) sum += val[q];
