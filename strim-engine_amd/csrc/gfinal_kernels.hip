@@ -1030,6 +1030,8 @@ __attribute__((not_tail_called)) __device__ __noinline__ XOut gfinal_rest(uint64
         cmd.bnd = ~0ull;
         cmd.bmp = ~0ull;
         int bz = -1, bfall = NOBIN;
+        bool crowded = false;  // the draw's bin, when it can be told, outgrows a zone
+        auto keys_of = [&](int bq) { return rcum.cnt(bq) - rcum.cnt(bq - 1); };
         uint64_t xw = 0ull;
         int xbn = NOBIN;
         if (step == 0) {
@@ -1072,6 +1074,8 @@ __attribute__((not_tail_called)) __device__ __noinline__ XOut gfinal_rest(uint64
               const int blo = rcum.find(true, (double)u_draw * (double)rcum.mass(bz - 1), bz + 1, 0ull, NOBIN);
               const int bhi = rcum.find(true, (double)u_draw * (double)rcum.mass(bz), bz + 1, 0ull, NOBIN);
               if (blo == bhi && blo <= bz) cmd.also = blo;
+              crowded = bhi - blo <= 1 && bhi <= bz && keys_of(blo) > (uint64_t)ZCAP &&
+                        keys_of(bhi) > (uint64_t)ZCAP;
             }
           }
           // (a Gumbel draw reads every kept token from the slots: it fails as soon as the
@@ -1081,21 +1085,24 @@ __attribute__((not_tail_called)) __device__ __noinline__ XOut gfinal_rest(uint64
               (step == glast && (bz >= rowfull || (by_rank && rcum.cnt(bz) > (uint64_t)ZCAP)))) {
             cmd.op = GOP_FAIL;
           } else if (zb[0] != bz && zb[1] != bz) {
+            const uint64_t cr = keys_of(bz);
             int full = rowfull;
             if (bz >= rowfull) {
               lists();
               full = listfull;
             }
-            if (bz >= full) {
+            // (a bin of more keys than a zone holds, this one or the draw's, is left to the
+            // exact resolution before anything is loaded for it)
+            if (cr > (uint64_t)ZCAP || crowded) {
+              cmd.op = GOP_FAIL;
+            } else if (bz >= full) {
               cmd.load = 2;
               cmd.also = -1;
             } else {
-              const uint64_t cr = rcum.cnt(bz) - rcum.cnt(bz - 1);
               const int also = cmd.also;
               const bool two = also >= 0 && also != bz && also < full &&
-                               cr + rcum.cnt(also) - rcum.cnt(also - 1) <= (uint64_t)GT;
+                               cr + keys_of(also) <= (uint64_t)GT;
               cmd.also = two ? also : -1;
-              if (cr > (uint64_t)ZCAP) cmd.op = GOP_FAIL;
               // lane c: chunk c's parts of the bins and their places in the zone
               const int bins[2] = {bz, cmd.also};
               int n[2];
