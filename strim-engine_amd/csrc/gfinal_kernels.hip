@@ -130,7 +130,7 @@ struct GFinalShared {
   int ii[GW];
   int misc[8];                    // 0 rowfull, 1 rowwin, 2 collect count, 3 some tail, 4 token,
                                   // 5 the leader's verdict, 6 a crowded bin (rank noise)
-  uint64_t res[2][4];             // a pick: key, count before, mass before, mass (two
+  uint64_t res[2][3];             // a pick: key, mass before, mass (two
   int32_t tag[2];                 // slots, alternating; tag = the pick's number)
   int zpo[2][LW], zpc[2][LW], zpz[2][LW];  // a zone's parts per chunk: first
                                                     // slot, count, place in the zone
@@ -154,10 +154,10 @@ __device__ __forceinline__ int row_bin(float arow, float l) {
   return d < (float)NBW ? (int)d : NOBIN;
 }
 
-// A pick: the key (~0: none), the count and mass of the keys before it in the row's
-// order, and its own mass.
+// A pick: the key (~0: none), the mass of the keys before it in the row's order, and its
+// own mass.
 struct GHit {
-  uint64_t key, cnt_before, mass_before, mass;
+  uint64_t key, mass_before, mass;
 };
 
 // The row's cumulative histogram in a wave's registers: lane l holds bins LPL l + q.
@@ -269,15 +269,14 @@ __device__ __forceinline__ GHit pick_rank(GFinalShared<LW>& S, GBig<LW>& G, int 
     const uint64_t own = by_mass ? (in ? km : 0ull) : 1ull;
     if (own > 0ull && (double)before <= thr && (double)(before + own) > thr) {
       S.res[slot][0] = k;
-      S.res[slot][1] = cnt0 + rank;
-      S.res[slot][2] = mass0 + mb;
-      S.res[slot][3] = km;
+      S.res[slot][1] = mass0 + mb;
+      S.res[slot][2] = km;
       S.tag[slot] = np;
     }
   }
   __syncthreads();
-  if (S.tag[slot] != np) return GHit{~0ull, 0ull, 0ull, 0ull};
-  return GHit{S.res[slot][0], S.res[slot][1], S.res[slot][2], S.res[slot][3]};
+  if (S.tag[slot] != np) return GHit{~0ull, 0ull, 0ull};
+  return GHit{S.res[slot][0], S.res[slot][1], S.res[slot][2]};
 }
 
 // The same pick over a zone of up to ZCAP keys at z0 (unsorted), for zones too wide for
@@ -319,11 +318,11 @@ __device__ __forceinline__ GHit pick_sorted(GFinalShared<LW>& S, GBig<LW>& G, in
   uint64_t pmask = ~((2ull << (hb < 0 ? 0 : hb)) - 1ull);  // the bits every candidate shares
   if (hb < 0) pmask = ~0ull;
   uint64_t prefix = ref & pmask;
-  uint64_t bc = cnt0, bm = mass0;  // weights below the candidates
+  uint64_t bc = cnt0, bm = mass0;  // weights below the candidates (bc: by count alone)
   while (hb >= 0) {
     const int shift = hb >= 7 ? hb - 7 : 0;
     const int copy = (lane & 1) << 8;
-    S.prk[t] = 0u;  // (two copies of 256 digits)
+    if (!by_mass) S.prk[t] = 0u;  // (two copies of 256 digits)
     S.pmb[t] = 0ull;
     __syncthreads();
 #pragma unroll
@@ -342,7 +341,7 @@ __device__ __forceinline__ GHit pick_sorted(GFinalShared<LW>& S, GBig<LW>& G, in
       uint64_t lm = 0ull;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        c[i] = S.prk[4 * lane + i] + S.prk[256 + 4 * lane + i];
+        c[i] = by_mass ? 0u : S.prk[4 * lane + i] + S.prk[256 + 4 * lane + i];
         mm[i] = S.pmb[4 * lane + i] + S.pmb[256 + 4 * lane + i];
         lc += c[i];
         lm += mm[i];
@@ -376,7 +375,7 @@ __device__ __forceinline__ GHit pick_sorted(GFinalShared<LW>& S, GBig<LW>& G, in
     }
     __syncthreads();
     const int d = S.ii[0];
-    if (d < 0) return GHit{~0ull, 0ull, 0ull, 0ull};  // (uniform) no key crosses
+    if (d < 0) return GHit{~0ull, 0ull, 0ull};  // (uniform) no key crosses
     prefix |= (uint64_t)d << shift;
     pmask |= 255ull << shift;
     bc = S.u2[0];
@@ -442,15 +441,14 @@ __device__ __forceinline__ GHit pick_sorted(GFinalShared<LW>& S, GBig<LW>& G, in
         const uint64_t own = by_mass ? kin : 1ull;
         if (lane < left && own > 0ull && (double)wb <= thr && (double)(wb + own) > thr) {
           S.res[slot][0] = k;
-          S.res[slot][1] = bc + rk;
-          S.res[slot][2] = bm + mb;
-          S.res[slot][3] = mk;
+          S.res[slot][1] = bm + mb;
+          S.res[slot][2] = mk;
           S.tag[slot] = np;
         }
       }
       __syncthreads();
-      if (S.tag[slot] != np) return GHit{~0ull, 0ull, 0ull, 0ull};
-      return GHit{S.res[slot][0], S.res[slot][1], S.res[slot][2], S.res[slot][3]};
+      if (S.tag[slot] != np) return GHit{~0ull, 0ull, 0ull};
+      return GHit{S.res[slot][0], S.res[slot][1], S.res[slot][2]};
     }
     const uint64_t vary = vo & va & ~pmask;
     hb = vary ? 63 - __clzll((long long)vary) : -1;
@@ -464,14 +462,13 @@ __device__ __forceinline__ GHit pick_sorted(GFinalShared<LW>& S, GBig<LW>& G, in
     if (ck[q] == prefix) {
       const int pos = t + GT * q;
       S.res[slot][0] = G.z.zkey[z0 + pos];
-      S.res[slot][1] = bc;
-      S.res[slot][2] = bm;
-      S.res[slot][3] = km[q];
+      S.res[slot][1] = bm;
+      S.res[slot][2] = km[q];
       S.tag[slot] = np;
     }
   __syncthreads();
-  if (S.tag[slot] != np) return GHit{~0ull, 0ull, 0ull, 0ull};
-  return GHit{S.res[slot][0], S.res[slot][1], S.res[slot][2], S.res[slot][3]};
+  if (S.tag[slot] != np) return GHit{~0ull, 0ull, 0ull};
+  return GHit{S.res[slot][0], S.res[slot][1], S.res[slot][2]};
 }
 
 // Sum of the masses of the zone's keys <= bound, zone zkey/zmass[z0, z0 + n) (every
@@ -1748,7 +1745,7 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
             Bm += mm[i];
           }
           const uint64_t bal = __ballot(hit >= 0);
-          if (bal == 0ull) return GHit{~0ull, 0ull, 0ull, 0ull};
+          if (bal == 0ull) return GHit{~0ull, 0ull, 0ull};
           const int hl = (int)__ffsll((long long)bal) - 1;
           const int d = __builtin_amdgcn_readlane(hit, hl);
           bc = rl_u64(hc, hl);
@@ -1778,11 +1775,11 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
         for (int q = 0; q < SQ; ++q)
           if (ck[q] == prefix) hq = q;
         const uint64_t bal = __ballot(hq >= 0);
-        if (bal == 0ull) return GHit{~0ull, 0ull, 0ull, 0ull};
+        if (bal == 0ull) return GHit{~0ull, 0ull, 0ull};
         const int hl = (int)__ffsll((long long)bal) - 1;
         const int q = __builtin_amdgcn_readlane(hq, hl);
         const uint64_t key = G.z.zkey[z0 + hl + WAVE * q], kmass = G.z.zmass[z0 + hl + WAVE * q];
-        return GHit{key, bc, bm, kmass};
+        return GHit{key, bm, kmass};
       };
       auto wpick = [&](int z0, int n, bool by_mass, double thr, uint64_t bnd, int excl,
                        uint64_t c0, uint64_t m0) -> GHit {
@@ -1824,10 +1821,9 @@ __global__ __launch_bounds__(GT) void k_gfinal(const ChunkStat* pre_cstat,
         const uint64_t own = by_mass ? kin : 1ull;
         const bool hit = mine && own > 0ull && (double)before <= thr && (double)(before + own) > thr;
         const uint64_t bal = __ballot(hit);
-        if (bal == 0ull) return GHit{~0ull, 0ull, 0ull, 0ull};
+        if (bal == 0ull) return GHit{~0ull, 0ull, 0ull};
         const int hl = (int)__ffsll((long long)bal) - 1;
-        return GHit{rl_u64(k, hl), c0 + (uint32_t)__builtin_amdgcn_readlane((int)rk, hl),
-                    m0 + rl_u64(mb, hl), rl_u64(km, hl)};
+        return GHit{rl_u64(k, hl), m0 + rl_u64(mb, hl), rl_u64(km, hl)};
       };
       // the zone's masses of keys <= bnd (n <= SOLO)
       auto wsum = [&](int z0, int n, uint64_t bnd) -> uint64_t {
