@@ -216,7 +216,8 @@ int strim_draft_argmax(void* stream, const void* draft_logits, int32_t dtype, in
  * when norm_weight is NULL); lm_head: bf16 [V][lm_head_stride]; out_logits: bf16
  * [B][out_stride]. xn[b][k] = bf16(w[k] * bf16(x[b][k] / sqrt(mean_k x^2 + eps))) (squares
  * summed in double), logits[b][v] = bf16(sum_k xn[b][k] lm_head[v][k]) accumulated in
- * float32 on MFMA. B in [1, 64]; K a positive multiple of 256; hidden, xn, lm_head and
+ * float32 on MFMA, in an order that K alone fixes: a row's logits are the same bits in
+ * every batch and with every V. B in [1, 64]; K a positive multiple of 256; hidden, xn, lm_head and
  * their row strides 16-byte aligned. Sizes or alignment out of range: STRIM_EINVAL. */
 int strim_head_logits(void* stream, const void* hidden, int64_t hidden_stride, int32_t B,
                       int32_t K, const void* norm_weight, float eps, void* xn,
@@ -226,8 +227,8 @@ int strim_head_logits(void* stream, const void* hidden, int64_t hidden_stride, i
 /* Hidden -> greedy token: the producer above (same operands and checks) with the pick
  * fused into it, for rows the reference decides by argmax alone (T <= 0 with no
  * penalties, no mask and no filters: Sampler.sample / SpecSampling's T -> 0 case,
- * SpecSampling.swift:70-88). The GEMV's epilogue writes each 128-row vocabulary tile's
- * first maximum per batch row (as bf16 logits, as strim_sample reads them) and one small
+ * SpecSampling.swift:70-88). The GEMV's epilogue writes each vocabulary tile's (32 to 128
+ * rows) first maximum per batch row (as bf16 logits, as strim_sample reads them) and one small
  * launch merges them, so the logits are not read back; out_logits may be NULL (then they
  * are not written at all). out_ids [B] = the first maximum's id, out_status [B] (or NULL)
  * = STRIM_OK, STRIM_ENONFINITE (a NaN or +inf logit) or STRIM_EEMPTY (every logit -inf),

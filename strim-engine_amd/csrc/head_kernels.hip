@@ -4,13 +4,14 @@
 //
 // k_head_norm: one workgroup per row, xn = bf16(w * bf16(x * inv)) with
 //   inv = 1 / sqrt(mean(x^2) + eps), the squares summed in double.
-// k_head_split (up to 16 rows, and more on small vocabularies), k_head_gemv (the others):
+// k_head_split (most calls of up to 16 rows, and more rows on small vocabularies),
+// k_head_gemv (the others; launch_head has the lines):
 //   logits[b][v] = bf16(sum_k xn[b][k] W[v][k]) with float accumulation. The weight matrix
 //   is read exactly once per call whatever the batch, which is the MFMA's N side (16 rows
 //   per tile, up to four tiles). k_head_split: a workgroup owns 32 or 64 vocabulary rows and
 //   its waves split K; the batch operand comes from the L2-resident xn. k_head_gemv: a
 //   workgroup owns 128 vocabulary rows, each wave two 16-row tiles over the whole of K,
-//   and the workgroup stages xn in LDS.
+//   and the workgroup stages xn in LDS. Both add a logit's products in one order (head_segs).
 //   For a greedy pick (strim_head_greedy) its epilogue also writes each batch row's first
 //   maximum over the workgroup's logits (as bf16 values, as the sampler reads them),
 //   and the logits may be left unwritten.
@@ -35,6 +36,12 @@ constexpr int HN_T = 1024;              // k_head_norm threads
 constexpr int HG_W = 4;                 // k_head_gemv waves per workgroup
 constexpr int HG_MT = 2;                // 16-row vocabulary tiles per wave
 constexpr int HG_KS = 128;              // K elements per step (four MFMAs of K 32)
+
+// Every kernel adds a logit's products in one order, which K alone fixes: K's n steps fall
+// into head_segs(K) segments, segment i the steps [i n / S, (i + 1) n / S); each segment is
+// one accumulator chain from zero, and the segments' sums are added in order. So a row's
+// logits are the same bits whatever the batch and the vocabulary it is computed with.
+constexpr int head_segs(int K) { return K >= 4096 ? 8 : 4; }
 
 // Round to nearest even; NaN stays a quiet NaN.
 __device__ __forceinline__ uint16_t head_bf16(float f) {
@@ -119,7 +126,7 @@ __device__ __forceinline__ void head_store4(uint16_t* dst, const uint16_t* o, in
 // NaN or +inf), id}; out NULL: no logits stored. MT: 16-row vocabulary tiles per wave; NW:
 // waves per workgroup.
 template <int NT, bool VO, bool TB, int MT, int NW>
-__global__ __launch_bounds__(NW* WAVE) void k_head_gemv(const uint16_t* xn, int64_t xn_stride,
+__global__ __launch_bounds__(NW* WAVE, NT == 2 ? 4 : 1) void k_head_gemv(const uint16_t* xn, int64_t xn_stride,
                                                           int B, int K, const uint16_t* W,
                                                           int64_t w_stride, int V,
                                                           uint16_t* out, int64_t out_stride,
@@ -134,11 +141,21 @@ __global__ __launch_bounds__(NW* WAVE) void k_head_gemv(const uint16_t* xn, int6
     const int v = min(v0 + mt * 16 + r16, V - 1);
     arow[mt] = W + (int64_t)v * w_stride + 8 * h;
   }
-  f32x4_t acc[MT][NT];
+  // the current segment's sums, and the finished segments': two batch tiles keep those in
+  // LDS (each thread its own) and four waves a SIMD (B = 24, V = 151,936, K = 5,120: 287.7 us,
+  // 291.1 with the registers at three waves, 297.8 with them at four; one chain over the whole
+  // of K, without the segments, 288.3)
+  constexpr bool LT = NT == 2;
+  __shared__ f32x4_t s_tot[LT ? MT * NT : 1][LT ? NW * WAVE : 1];
+  f32x4_t acc[MT][NT], tot[LT ? 1 : MT][LT ? 1 : NT];
+  auto total = [&](int mt, int nt) -> f32x4_t& {
+    if constexpr (LT) return s_tot[mt * NT + nt][threadIdx.x];
+    else return tot[mt][nt];
+  };
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = total(mt, nt) = f32x4_t{0.f, 0.f, 0.f, 0.f};
   // two register buffers: the next step's loads are in flight while this step multiplies
   uint4 a[2][MT][4];
   auto loada = [&](int buf, int kb) {
@@ -151,7 +168,23 @@ __global__ __launch_bounds__(NW* WAVE) void k_head_gemv(const uint16_t* xn, int6
   // unconditional (the last prefetch reloads the last step and is not used), and the
   // scheduling barriers keep each buffer's loads issued before the other buffer's
   // multiplies: left alone, the compiler sinks the loads next to their use
-  const int nsteps = K / HG_KS;
+  const int nsteps = K / HG_KS, segs = head_segs(K);
+  int seg = 1, seg_end = nsteps / segs;
+  // after `done` steps: a finished segment's sums join the total (a segment may be empty)
+  auto end_step = [&](int done) {
+    if (done < seg_end || done == nsteps) return;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) {
+        total(mt, nt) += acc[mt][nt];
+        acc[mt][nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      }
+    do {
+      ++seg;
+      seg_end = seg * nsteps / segs;
+    } while (seg_end <= done);
+  };
   // Several batch tiles: every wave needs the same 16 NT rows of xn at each step, so
   // the workgroup stages them in LDS once (double-buffered, rows padded by 16 bytes so
   // the 16 rows a wave reads fall in different banks) instead of each wave reading
@@ -213,6 +246,7 @@ __global__ __launch_bounds__(NW* WAVE) void k_head_gemv(const uint16_t* xn, int6
     loada(1, (s + 1) * HG_KS);
     __builtin_amdgcn_sched_barrier(0);
     mma_lds(0, 0);
+    end_step(s + 1);
     __builtin_amdgcn_sched_barrier(0);
     xstore(1, x1);
     sync_lds();
@@ -221,10 +255,15 @@ __global__ __launch_bounds__(NW* WAVE) void k_head_gemv(const uint16_t* xn, int6
     loada(0, s2);
     __builtin_amdgcn_sched_barrier(0);
     mma_lds(1, 1);
+    end_step(s + 2);
     __builtin_amdgcn_sched_barrier(0);
     xstore(0, x0);
     sync_lds();
   }
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = total(mt, nt) + acc[mt][nt];
   // lane l holds rows 4 h + i of each tile for batch row nt 16 + r16
   float bv[NT];
   int bi[NT];
@@ -293,10 +332,11 @@ __global__ __launch_bounds__(NW* WAVE) void k_head_gemv(const uint16_t* xn, int6
 
 // The same product with K split over the workgroup's waves: wave w multiplies the steps
 // [w n / NW, (w + 1) n / NW) of the same MT 16-row tiles, and the partial sums are added in
-// wave order through LDS. Bound by HBM. A workgroup that holds 128 rows over the whole of K
-// leaves the chip half empty at its end, or throughout where V / 128 is near or below the
-// 256 CUs; K / NW on 32 rows makes pieces a sixteenth the size (each wave's batch slice
-// is read from L2 either way at one batch tile). B = 8, K = 5,120: 109.6 -> 77.8 us at
+// wave order through LDS (NW = head_segs(K): a wave's steps are one segment). Bound by HBM. A
+// workgroup that holds 128 rows over the whole of K leaves the chip half empty at its end,
+// or throughout where V / 128 is near or below the 256 CUs; 32 rows are a quarter of its
+// work, and a wave does a quarter (four waves) or an eighth (eight) of what one of its four
+// waves did (each wave's batch slice is read from L2 either way at one batch tile). B = 8, K = 5,120: 109.6 -> 77.8 us at
 // V = 40,000 (65 at a plain read's 6.26 TB/s), 54.4 -> 21.6 at V = 8,192, 280.0 -> 272.8 at
 // V = 151,936; K = 2,048, V = 151,936: 143.5 -> 109.7.
 template <int NT, bool VO, bool TB, int MT, int NW>
@@ -495,7 +535,7 @@ hipError_t launch_head(const void* hidden, int64_t hidden_stride, int B, int K,
   // B = 24 36.9 -> 30.7, B = 64 42.9 against 47.1).
   const int nt = (B + 15) / 16;
   const bool split = nt == 1 || V <= (nt == 2 ? 14336 : 9216);
-  const bool deep = nt == 1 && K >= 4096, tall = deep && B >= 11 && V >= 65536;
+  const bool deep = head_segs(K) == 8, tall = nt == 1 && deep && B >= 11 && V >= 65536;
   const int rows = split ? (tall ? 64 : 32) : HG_W * HG_MT * 16;
   const dim3 grid((unsigned)((V + rows - 1) / rows));
 #define STRIM_HEAD_(K_, NT_, MT_, NW_, VO_, TB_)                                              \
@@ -510,10 +550,12 @@ hipError_t launch_head(const void* hidden, int64_t hidden_stride, int B, int K,
     else STRIM_HEAD_(K_, NT_, MT_, NW_, false, false);            \
   } while (0)
   if (tall) STRIM_HEAD(k_head_split, 1, 4, 8);
-  else if (deep) STRIM_HEAD(k_head_split, 1, 2, 8);
+  else if (nt == 1 && deep) STRIM_HEAD(k_head_split, 1, 2, 8);
   else if (nt == 1) STRIM_HEAD(k_head_split, 1, 2, 4);
+  else if (nt == 2 && split && deep) STRIM_HEAD(k_head_split, 2, 2, 8);
   else if (nt == 2 && split) STRIM_HEAD(k_head_split, 2, 2, 4);
   else if (nt == 2) STRIM_HEAD(k_head_gemv, 2, HG_MT, HG_W);
+  else if (split && deep) STRIM_HEAD(k_head_split, 4, 2, 8);
   else if (split) STRIM_HEAD(k_head_split, 4, 2, 4);
   else STRIM_HEAD(k_head_gemv, 4, HG_MT, HG_W);
 #undef STRIM_HEAD

@@ -60,7 +60,10 @@ def test_head_logits_match_fp64_product(B, K, V):
                                        (11, 4096, 65537, 0), (16, 5120, 65600, 1),
                                        (17, 256, 14336, 0), (32, 768, 14335, 1),
                                        (17, 256, 14337, 0), (33, 256, 9216, 0), (64, 1280, 9215, 1),
-                                       (33, 256, 9217, 0)])
+                                       (33, 256, 9217, 0), (9, 4352, 65536, 0), (10, 4352, 65536, 0),
+                                       (10, 6144, 65536, 0), (11, 4096, 65536, 0),
+                                       (11, 4352, 70000, 0), (16, 4352, 70000, 1),
+                                       (24, 4096, 8200, 0), (40, 4352, 8200, 3)])
 def test_head_split_forms(B, K, V, pad):
     """K split over a workgroup's waves: fewer steps than waves, step counts that the waves do
     not share evenly, row tiles past the vocabulary, and both sides of each line of the
@@ -93,6 +96,26 @@ def test_head_split_forms(B, K, V, pad):
     assert (st.cpu().numpy() == 0).all()
     np.testing.assert_array_equal(ids.cpu().numpy(), np.argmax(to_np(out), axis=1))
     c.close()
+
+
+@pytest.mark.parametrize("K", [256, 1280, 3840, 4096, 4352, 5120, 8192])
+def test_head_row_bits_do_not_depend_on_the_call(K):
+    """A hidden row's logits are the same bits in every batch and with every vocabulary it is
+    computed with: each form of the producer (both sides of each line of the dispatch) adds
+    the products in the same order. Values spread over many exponents, so that another order
+    would round differently."""
+    print(f"[head] row bits K={K}", flush=True)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(K)
+    V = 65_600
+    x = torch.randn(64, K, device="cuda", generator=g)
+    x = (x * torch.exp(2.0 * torch.randn(64, K, device="cuda", generator=g))).to(torch.bfloat16)
+    W = (0.05 * torch.randn(V, K, device="cuda", generator=g)).to(torch.bfloat16)
+    ref = torch.cat([ops.head_logits(x[b:b + 1], W[:4096]) for b in range(64)])
+    for Vs in (65_536, V, 14_337, 14_336, 9217, 9216, 8200, 4096):
+        for B in (1, 2, 9, 10, 11, 16, 17, 32, 33, 64):
+            out = ops.head_logits(x[:B], W[:Vs])
+            assert torch.equal(out[:, :4096], ref[:B]), f"V={Vs} B={B}"
 
 
 def test_head_logits_no_norm_and_strided_output():
