@@ -537,21 +537,32 @@ hipError_t launch_head(const void* hidden, int64_t hidden_stride, int B, int K,
     src = (const uint16_t*)xn;
     src_stride = K;
   }
-  // One batch tile: always split. K from 4,096 (four steps and more a wave) over eight
-  // waves, else four (B = 8, V = 151,936: 272.8 against 275.8 us at K = 5,120, 117.5 against
-  // 109.7 at K = 2,048). 64 rows a workgroup, in place of 32, halve the reads of xn, which
-  // count where its tile's rows are distinct and the vocabulary still fills the chip
-  // (K = 5,120, B = 16: 303 against 317 us at V = 151,936, 157 against 169 at 80,000, but
-  // 92.6 against 89.2 at 40,000; B = 8, V = 151,936: 284 against 273; B = 11, V = 65,536:
-  // 124.1 against 127.4).
+  // One batch tile: K split over eight waves where it has eight segments (head_segs), else
+  // four. 32 vocabulary rows a workgroup; at K from 4,096, two forms read xn less often,
+  // which counts where its tile's rows are distinct: 64 rows a workgroup, and the staged
+  // kernel (its build for two tiles). Both take their time in whole rounds over the 256
+  // CUs, of 16,384 and 32,768 rows, so they are for vocabularies that nearly fill their
+  // last round, the more nearly the fewer rows there are. K = 5,120, us for 32 rows, 64
+  // rows, staged: V = 151,936 (rounds 93 % full) B = 10 286 289 279, B = 16 315 302 284;
+  // V = 65,536 (full) B = 10 125.0 123.0 118.1; V = 80,000 (98 and 81 %) B = 12 161 153
+  // 164; V = 100,000 (87 and 76 %) B = 12 201 206 215, B = 16 213 210 217. Where K is a
+  // multiple of 2,048 the staged kernel's rows meet in few memory channels (K = 6,144,
+  // V = 131,072, B = 16: 299 300 325; K = 8,192, V = 128,256: 432 385 451).
   // More tiles: the staged slice of xn is worth more than the split, until its 128-row
   // workgroups leave most CUs idle (its time hardly falls below V = 20,000, the split's is
   // in proportion to V. K = 5,120, V = 8,192: B = 24 50.4 -> 26.5 us, B = 64 59.1 -> 37.8;
   // V = 20,000: B = 24 56.1 against 62.0, B = 64 65 against 97; K = 3,584, V = 10,672:
   // B = 24 36.9 -> 30.7, B = 64 42.9 against 47.1).
-  const int nt = (B + 15) / 16;
+  const bool deep = head_segs(K) == 8;
+  auto fills = [&](int unit) {  // the rounds of `unit` rows are (103 - B) % full or more
+    const int64_t rounds = ((int64_t)V + unit - 1) / unit;
+    return 100 * (int64_t)V >= (103 - B) * unit * rounds;
+  };
+  const bool wide1 = B <= 16 && deep && V >= 65536;
+  const bool staged1 = wide1 && B >= 10 && K % 2048 != 0 && fills(32768);
+  const bool tall = wide1 && !staged1 && B >= 11 && fills(16384);
+  const int nt = staged1 ? 2 : (B + 15) / 16;
   const bool split = nt == 1 || V <= (nt == 2 ? 14336 : 9216);
-  const bool deep = head_segs(K) == 8, tall = nt == 1 && deep && B >= 11 && V >= 65536;
   const int rows = split ? (tall ? 64 : 32) : HG_W * HG_MT * 16;
   const dim3 grid((unsigned)((V + rows - 1) / rows));
 #define STRIM_HEAD_(K_, NT_, MT_, NW_, VO_, TB_)                                              \
