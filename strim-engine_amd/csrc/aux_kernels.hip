@@ -24,17 +24,22 @@ __global__ __launch_bounds__(256) void k_mask_logits(const void* logits, int dty
 // MTP.nextTokenIndex (Sources/StrimCore/MTP.swift:104-111): argMax over the truncated
 // draft vocab (first max), then the draft->full index table.
 //
-// One 1024-thread workgroup per row: a row is at most a few hundred KB, so its time is
-// the memory round trip and the reduction, and a merge across workgroups would cost a
-// second launch. A thread takes its batch's 16-byte loads in flight (32 tokens; the whole of a
-// 32,768-token row in one batch for either dtype). At R = 4, Vd = 32,768 bf16 the kernel
-// takes 4.2 us against 27.7 us with 256 threads of 2-byte loads, one in flight.
+// One workgroup per row: a row is at most a few hundred KB, so its time is the memory round
+// trip and the reduction, and a merge across workgroups would cost a second launch. T
+// threads with the 16-byte loads of N tokens each in flight (a batch): 1,024 threads of 32
+// tokens take a 32,768-token row of either dtype in one (R = 4, bf16: 4.0 us against 27.7
+// with 256 threads of 2-byte loads, one in flight). Rows of up to DA_SMALL tokens, and past
+// DA_ROWS rows those of up to 4 DA_SMALL, take 256 threads of 8: a short row has no work for
+// more, and many rows share the CUs (us, bf16, 1,024 threads against 256: R = 4, Vd = 1,001
+// unaligned 4.7 and 2.8, 4,096 3.2 and 3.1, 16,384 3.6 and 4.8; R = 4,096, Vd = 4,096 20.6 and
+// 8.0, 16,384 28.2 and 22.6).
 // VEC: rows 16-byte aligned; other rows load token by token, in batches as wide.
-constexpr int DA_T = 1024, DA_N = 32;  // threads, tokens a thread and batch
-template <bool BF16, bool VEC>
-__global__ __launch_bounds__(DA_T) void k_draft_argmax(const void* logits, int Vd,
-                                                       int64_t row_stride, const int32_t* table,
-                                                       int32_t* out) {
+constexpr int DA_SMALL = 4096, DA_ROWS = 512;
+template <bool BF16, bool VEC, int T, int N>
+__global__ __launch_bounds__(T) void k_draft_argmax(const void* logits, int Vd,
+                                                    int64_t row_stride, const int32_t* table,
+                                                    int32_t* out) {
+  constexpr int DA_T = T, DA_N = N;
   __shared__ float s_v[DA_T / WAVE];
   __shared__ int s_i[DA_T / WAVE];
   const int r = blockIdx.x, t = threadIdx.x, lane = t & (WAVE - 1), w = wave_id();
@@ -123,14 +128,20 @@ __global__ __launch_bounds__(DA_T) void k_draft_argmax(const void* logits, int V
 hipError_t launch_draft_argmax(const void* logits, bool bf16, bool vec, int R, int Vd,
                                int64_t row_stride, const int32_t* table, int32_t* out,
                                hipStream_t st) {
-  const dim3 grid((unsigned)R), blk(DA_T);
-#define STRIM_DA(B_, V_)                                                                        \
-  hipLaunchKernelGGL((k_draft_argmax<B_, V_>), grid, blk, 0, st, logits, Vd, row_stride, table, \
-                     out)
-  if (bf16 && vec) STRIM_DA(true, true);
-  else if (bf16) STRIM_DA(true, false);
-  else if (vec) STRIM_DA(false, true);
-  else STRIM_DA(false, false);
+  const bool small = Vd <= DA_SMALL || (R > DA_ROWS && Vd <= 4 * DA_SMALL);
+#define STRIM_DA(B_, V_, T_, N_)                                                              \
+  hipLaunchKernelGGL((k_draft_argmax<B_, V_, T_, N_>), dim3((unsigned)R), dim3(T_), 0, st,    \
+                     logits, Vd, row_stride, table, out)
+#define STRIM_DA_(B_, V_)                \
+  do {                                   \
+    if (small) STRIM_DA(B_, V_, 256, 8); \
+    else STRIM_DA(B_, V_, 1024, 32);     \
+  } while (0)
+  if (bf16 && vec) STRIM_DA_(true, true);
+  else if (bf16) STRIM_DA_(true, false);
+  else if (vec) STRIM_DA_(false, true);
+  else STRIM_DA_(false, false);
+#undef STRIM_DA_
 #undef STRIM_DA
   return hipGetLastError();
 }

@@ -89,8 +89,7 @@ def test_sweep_large_batch(ctx, V):
 def test_vocab_past_64_chunks(V):
     # rows at and past the lattice's 40 chunks (163,840 tokens) and past 64 chunks (up to
     # the 2^20 maximum): up to 64 chunks every wave reduces the chunk statistics alone,
-    # past that they merge across waves; general rows past 40 chunks take the exact
-    # resolution
+    # past that they merge across waves, and general rows take the exact resolution
     rng = np.random.default_rng(V % 1000)
     B = 4
     x = rng.normal(0, 2.0, size=(B, V)).astype(np.float32)
@@ -327,8 +326,8 @@ def test_rank_noise_wide_nucleus(ctx, injected):
 def test_wide_nuclei_window_lists(V, B, dtype):
     """Nuclei past the chunks' slots, whose cut or draw bin is gathered from the window
     lists: top-p, large top-k and no filter, masks, tied values, aligned and odd rows, one
-    chunk and many, rows without a list in the same batch (peaked, penalised, past the 64
-    rows of a group), and bins past a zone's capacity (the exact resolution)."""
+    chunk and many, several groups of rows, rows without a list in the same batch (peaked,
+    penalised), and bins past a zone's capacity (the exact resolution)."""
     rng = np.random.default_rng(V + B)
     x = rng.normal(0, 1.0, size=(B, V)).astype(np.float32)
     x[1] *= 2.0
@@ -348,6 +347,24 @@ def test_wide_nuclei_window_lists(V, B, dtype):
     check_sample(c, x, p, dtype, mask=mask, noise=noise, probs=False, label=f"wide masked V={V} B={B}")
     p["presence_penalty"] = np.resize([0.0, 0.5], B)
     check_sample(c, x, p, dtype, history=hist, noise=noise, probs=False, label=f"wide pen V={V} B={B}")
+    c.close()
+
+
+@pytest.mark.parametrize("B,k,V", [(20, 3, 20003), (33, 1, 9001), (9, 7, 40001)])
+def test_wide_nuclei_past_the_listed_rows(B, k, V):
+    """A verify launch of more than 64 rows over wide nuclei: the window lists have room for
+    the first 64 rows of a launch, and the rows past them take the collect pass."""
+    rng = np.random.default_rng(V + B)
+    x = rng.normal(0, 1.0, size=(B, k + 1, V)).astype(np.float32)
+    drafts = x[:, :k].argmax(-1).astype(np.int32)
+    drafts[::2] = rng.integers(0, V, size=drafts[::2].shape)
+    p = O.make_params(B, top_p=np.resize([0.95, 0.9, 0.97], B),
+                      seed=rng.integers(0, 2**63, size=B, dtype=np.uint64), position=4)
+    c = ops.Context(0, max_rows=B * (k + 1), max_vocab=V)
+    say(f"wide nuclei past the listed rows B={B} k={k} V={V}")
+    for dtype in ("bf16", "f32"):
+        check_verify(c, x, k, drafts, p, dtype, noise_mode=O.NOISE_ICDF,
+                     noise=rng.random((B, k + 1, 2), dtype=np.float32), label="past 64 rows")
     c.close()
 
 
@@ -799,7 +816,9 @@ def test_draft_argmax(ctx):
 
 # ------------------------------------------------------------ mirror API ----
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
-@pytest.mark.parametrize("Vd,stride", [(1, 1), (3, 3), (7, 8), (8, 8), (1001, 1001), (32767, 32768),
+@pytest.mark.parametrize("Vd,stride", [(1, 1), (3, 3), (7, 8), (8, 8), (1001, 1001), (2047, 2048),
+                                       (2049, 2056), (4095, 4096), (4096, 4096), (4097, 4104),
+                                       (4099, 4099), (32767, 32768),
                                        (32768, 32768), (32769, 32784), (70003, 70008)])
 def test_draft_argmax_forms(dtype, Vd, stride):
     """Rows at the edges of a load and of a batch, aligned and unaligned, with ties (first
@@ -828,6 +847,17 @@ def test_draft_argmax_forms(dtype, Vd, stride):
         np.testing.assert_array_equal(ops.draft_argmax(base, dev(table)).cpu().numpy(), table[exp])
         one = ops.draft_argmax(base[2])
         assert int(one.item()) == exp[2]
+
+
+@pytest.mark.parametrize("R", [512, 513])
+@pytest.mark.parametrize("Vd", [4096, 4097, 16384, 16385])
+def test_draft_argmax_many_rows(R, Vd):
+    """Both sides of the lines between the two workgroup sizes, with ties (first maximum)."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(R + Vd)
+    x = torch.randn(R, Vd, device="cuda", generator=g).to(torch.bfloat16)
+    first = (x == x.amax(1, keepdim=True)).int().argmax(1)
+    torch.testing.assert_close(ops.draft_argmax(x).long(), first, rtol=0, atol=0)
 
 
 def test_sampler_mirror_matches_oracle(ctx):
