@@ -156,8 +156,11 @@ struct ExactReq {
 // Decides a row whose candidates overflow the finalize by the exact streaming resolution
 // (all threads of the workgroup call it). Out of line, with the launch's fields and the
 // row's parameters read again: held for it, they took scalar registers from the common
-// path (75 scalar spills to vector lanes, 25 without: B = 1 top-k 14.4 -> 14.1 us a call,
-// the unfiltered one-hot verify 23.0 -> 22.6). GQ: see k_finalize.
+// path (75 scalar spills to vector lanes, 25 without; call times within 2 % either way).
+// General-q draft rows run it here, 256 threads beside each other, where k_final would take
+// 1,024 a row after this launch: with every row of a sequence past its candidates, B = 4,
+// k = 3, V = 151,936, min-p 0.01 and top-p 0.95, 1,366 against 1,721 us a round; with the
+// bonus row alone decided from its candidates 1,369 against 1,149. GQ: see k_finalize.
 template <bool GQ>
 __attribute__((not_tail_called)) __device__ __noinline__ void finalize_exact(
     uint64_t kargs, int r, const ExactReq q_in, lds_t<FinalShared>* Sl) {

@@ -14,11 +14,12 @@
 //   2. the bin's tokens (its zone), gathered from the chunks' slot regions (each chunk's
 //      part of the bin is a contiguous run there) and resolved exactly in (l desc, id asc)
 //      order, each token's mass taken from its own l.
-// A zone in a bin that some chunk could not write whole is collected by one streaming
-// pass of this workgroup over the row. A decision below a chunk's window (the lattice
-// cannot place it), rank-indexed noise over more tokens than a zone holds and rows whose
-// lattice words were not written take
-// the exact streaming resolution (exact.hpp).
+// A zone in a bin that some chunk could not write whole is gathered from the chunks' window
+// lists, or, where a chunk has no list, collected by one streaming pass of this workgroup
+// over the row. A decision below a chunk's window (the lattice cannot place it), a zone of
+// more than ZCAP keys, a Gumbel draw over a kept set that ends past the slots, rank-indexed
+// noise over more tokens than a zone holds and rows whose lattice words were not written
+// take the exact streaming resolution (exact.hpp).
 //
 // Masses are fixed point, 2^40 per unit of exp(l - m) (RFIX): integer sums make every
 // cumulative mass independent of summation order. A chunk's bin masses (2^37 per unit of
@@ -31,9 +32,8 @@
 // on the row's parameters are issued first, and the leader wave keeps the row's cumulative
 // histogram in its own registers (a decision's bin search needs no barrier). What the
 // leader does not decide alone is out of line (gfinal_rest): with it inline the common
-// path kept 258 scalar values in vector lanes, 11 without (8 constrained rows 20.1 -> 19.6
-// us a call; the wide-nucleus rows 97 -> 92.7, their calls reading the launch's fields by
-// scalar loads instead of copies in scratch memory).
+// path spilled 213 scalar registers to vector lanes, 14 without (8 constrained rows 20.1 ->
+// 19.6 us a call; a row that needs the call pays about 1.5 us for it).
 #include "exact.hpp"
 
 namespace strim {
@@ -50,8 +50,8 @@ constexpr int DW = GW - 1;  // the waves that load into LDS: all but wave 0
 // k_gfinal is built for rows of up to LW = 40 chunks (V <= 163,840) and up to LW = 64
 // (V <= 262,144): the LDS holds every chunk's lattice words, so the wider build keeps
 // fewer prefetched candidates a chunk (PF). Rows past 40 chunks took the exact resolution
-// before: B = 1, V = 248,320, top-p 0.95, rank-indexed Gumbel noise took 586 us a call and
-// takes 26.6. Both are built because a crowded bin's candidates lie past 56 a chunk more
+// before: B = 1, V = 248,320, top-p 0.95, rank-indexed Gumbel noise took 592 us a call and
+// takes 22 to 28. Both are built because a crowded bin's candidates lie past 56 a chunk more
 // often than past 160: the 8-row constrained step of 38 chunks takes 19.6 us, and 25.1 on
 // the wider build.
 template <int LW>
