@@ -631,7 +631,9 @@ __global__ __launch_bounds__(stpb<SSEG>()) void k_stream(const void* pre_logits,
           }
           const float keep = p.top_p < 1.0f ? p.top_p : 0.95f;
           t2 = p.top_p < 1.0f ? (uint32_t)((0.75f + 0.25f * keep) * 0x1p24f) : ~0u;
-          t1 = cs.n <= CHUNK / 4 ? t2 : (uint32_t)(0.9f * keep * 0x1p24f);
+          // (no margin where one chunk is most of the row: its own cut is near the row's)
+          const float margin = 3 * P.V < 4 * CHUNK ? 1.0f : 0.9f;
+          t1 = cs.n <= CHUNK / 4 ? t2 : (uint32_t)(margin * keep * 0x1p24f);
         }
 #pragma unroll
         for (int q = 0; q < LPL; ++q) sum += val[q];
